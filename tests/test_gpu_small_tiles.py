@@ -1,0 +1,135 @@
+"""GPU parity of the small-tile grouped GEMM (few rows per expert, few tiles).
+
+Cases sit at the edges of its choices: 64- and 128-row tiles, 128 and 256
+weight rows (the last tile half full), one row, a full tile and one row
+more, empty experts, k of one stage and of fewer stages than the ring, and
+rows a multiple of 4 KB apart (the k walk then starts elsewhere per tile).
+Tolerance: the inputs are bf16 and the sums fp32, so an output is off by
+its bf16 rounding (2^-9 relative, and the pre-activation's once more through
+the SwiGLU); 1e-2 of the row's largest value covers both.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import DEV, announce, assert_close, bf16_dev, f32_dev, rand_bf16, to_np
+from oracle import moe_oracle as O
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-2
+
+# rows per expert, N (or H for the SwiGLU: 2 H weight rows), K
+CASES = [
+    ((1,), 128, 64),                                 # one row, one k stage
+    ((0, 1, 0, 2, 1), 192, 2048),                    # 64 x 128 tiles, rotated k walk
+    ((64, 65, 33, 1, 0, 63), 320, 192),              # 64-row tiles and one row past
+    ((5,) * 300, 384, 320),                          # more than one round, fewer stages than the ring
+    ((9,) * 200 + (0,) * 20 + (64,) * 3, 1152, 256),   # 64 x 256 tiles, half-full last tile
+    ((128, 129, 97, 1, 300, 0, 31), 448, 384),       # 128 x 128 tiles, one row past
+    ((90, 100, 128, 70, 96) * 26, 1152, 2048),         # 128 x 256 tiles, whole and partial rounds, rotated
+    ((700, 1300), 640, 1024),                        # more rows per expert, tiles too few for the large kernel
+]
+
+
+def _case(i):
+    counts, n, k = CASES[i]
+    counts = np.array(counts, np.int64)
+    rng = np.random.default_rng(100 + i)
+    return counts, int(counts.sum()), len(counts), n, k, rng
+
+
+def _offs(counts):
+    return torch.from_numpy(np.cumsum(counts).astype(np.int32)).to(DEV)
+
+
+@pytest.mark.parametrize("i", range(len(CASES)))
+@pytest.mark.parametrize("limit", [None, 0.5])
+def test_small_swiglu(ops, i, limit):
+    counts, M, E, H, D, rng = _case(i)
+    T = (M + 1) // 2
+    tok, w13 = rand_bf16(rng, (T, D)), rand_bf16(rng, (E, 2 * H, D), 0.05)
+    src = rng.integers(0, 2 * T, M).astype(np.int32)
+    announce(f"small swiglu M={M} E={E} H={H} D={D} limit={limit}")
+    wd, od = bf16_dev(w13), _offs(counts)
+    h_ref = O.bf16_round(O.grouped_mm(tok[src // 2], w13, np.cumsum(counts)))
+    a_ref = O.swiglu(h_ref, limit)
+    a, h = ops.grouped_mm_swiglu(bf16_dev(tok[src // 2]), wd, od, limit, save_h=True)
+    assert_close(to_np(h), h_ref, TOL, "h")
+    assert_close(to_np(a), a_ref, 2 * TOL, "a")
+    if D >= 128:
+        a2, h2 = ops.grouped_mm_swiglu_gather(bf16_dev(tok), torch.from_numpy(src).to(DEV), 2, wd, od, limit, save_h=True)
+        assert torch.equal(a, a2) and torch.equal(h, h2), "gathered rows differ from the same rows given in order"
+
+
+@pytest.mark.parametrize("i", range(len(CASES)))
+def test_small_store_and_scatter(ops, i):
+    counts, M, E, N, K, rng = _case(i)
+    N = -(-N // 128) * 128
+    x, w = rand_bf16(rng, (M, K)), rand_bf16(rng, (E, N, K), 0.05)
+    dest = rng.permutation(M).astype(np.int32)
+    scale = rng.random(M).astype(np.float32)
+    announce(f"small store / scatter M={M} E={E} N={N} K={K}")
+    xd, wd, od = bf16_dev(x), bf16_dev(w), _offs(counts)
+    y = O.grouped_mm(x, w, np.cumsum(counts))
+    assert_close(to_np(ops.grouped_mm(xd, wd, od)), y, TOL, "store")
+    out = ops.grouped_mm_unpermute(xd, wd, od, f32_dev(scale), torch.from_numpy(dest).to(DEV), M)
+    ref = np.zeros((M, N), np.float32)
+    ref[dest] = y * scale[:, None]
+    assert_close(to_np(out), ref, TOL, "scatter")
+
+
+@pytest.mark.parametrize("T,D,H", [(1, 128, 64), (70, 256, 192), (900, 512, 448)])
+def test_small_shared_expert(ops, T, D, H):
+    """The accumulating, gated epilogue (one expert with every row)."""
+    rng = np.random.default_rng(T)
+    x, w13, w2 = rand_bf16(rng, (T, D)), rand_bf16(rng, (1, 2 * H, D), 0.05), rand_bf16(rng, (1, D, H), 0.05)
+    base, gate = rand_bf16(rng, (T, D)), rng.standard_normal(T).astype(np.float32)
+    announce(f"small shared expert T={T} D={D} H={H}")
+    out = ops.shared_expert_add(bf16_dev(base), bf16_dev(x), bf16_dev(w13[0]), bf16_dev(w2[0]), f32_dev(gate))
+    a = O.bf16_round(O.swiglu(O.bf16_round(O.grouped_mm(x, w13, np.array([T])))))
+    y = O.bf16_round(O.grouped_mm(a, w2, np.array([T])) / (1 + np.exp(-gate[:, None])))
+    assert_close(to_np(out), base + y, TOL, "out")
+
+
+def test_large_tiles_split_epilogues_and_replay(ops):
+    """35 experts of 320 rows keep the 320 x 256 kernel, whose 24 leftover
+    tiles (of 280) are cut along k: the SwiGLU epilogue (with and without the
+    gather) and the scatter one, and replays of the captured pair with other
+    work in between (the plan's arrival counters must return to zero)."""
+    E, D, H = 35, 2048, 1024
+    counts = np.full(E, 320)
+    M = int(counts.sum())
+    rng = np.random.default_rng(7)
+    labels = rng.permutation(np.repeat(np.arange(E), counts))
+    sidx = O.stable_order(labels, E).astype(np.int32)
+    x, w13 = rand_bf16(rng, (M, D)), rand_bf16(rng, (E, 2 * H, D), 0.05)
+    a, w2 = rand_bf16(rng, (M, 2048)), rand_bf16(rng, (E, D, 2048), 0.05)
+    scale = rng.random(M).astype(np.float32)
+    announce("large tiles, split swiglu gather / scatter, replayed")
+    xd, sd, od, ad, wd13, wd2 = (bf16_dev(x), torch.from_numpy(sidx).to(DEV), _offs(counts), bf16_dev(a),
+                                 bf16_dev(w13), bf16_dev(w2))
+
+    def step():
+        act, _ = ops.grouped_mm_swiglu_gather(xd, sd, 1, wd13, od)
+        return act, ops.grouped_mm_unpermute(ad, wd2, od, f32_dev_scale, sd, M)
+
+    f32_dev_scale = f32_dev(scale)
+    act, out = step()
+    plain, _ = ops.grouped_mm_swiglu(bf16_dev(x[sidx]), wd13, od)
+    assert torch.equal(act, plain)
+    h_ref = O.bf16_round(O.grouped_mm(x[sidx], w13, np.cumsum(counts)))
+    assert_close(to_np(act), O.swiglu(h_ref), 2 * TOL, "a")
+    ref = np.zeros((M, D), np.float32)
+    ref[sidx] = O.grouped_mm(a, w2, np.cumsum(counts)) * scale[:, None]
+    assert_close(to_np(out), ref, TOL, "out")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        g_act, g_out = step()
+    for _ in range(3):
+        g_act.zero_(), g_out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(g_act, act) and torch.equal(g_out, out)
+        step()

@@ -25,9 +25,7 @@ namespace ttamd {
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void tile_map_kernel(const int* __restrict__ offs, int E,
                                                         int M, int max_tiles, int max_rows,
-                                                        int4* __restrict__ table,
-                                                        int* __restrict__ count,
-                                                        int* __restrict__ split_cnt) {
+                                                        const TileTable t, int max_small) {
   __shared__ int sh[1024 / kWave + 1];
   auto range = [&](int e, int& r0, int& r1) {
     // offs == nullptr: one expert owning all M rows
@@ -36,13 +34,13 @@ __global__ __launch_bounds__(1024) void tile_map_kernel(const int* __restrict__ 
     r0 = min(max(a, 0), M);
     r1 = min(max(b, r0), M);
   };
-  block_tile_table<1024>(range, E, max_tiles, max_rows, table, count, split_cnt, sh);
+  block_tile_plan<1024>(range, E, max_tiles, max_rows, t, max_small, sh);
 }
 
-hipError_t launch_tile_map(const int* offs, int E, int M, int max_rows, void* ws, hipStream_t stream) {
-  TileTable tt = tile_table_in(ws);
+hipError_t launch_tile_map(const int* offs, int E, int M, int max_rows, void* ws, bool with_small,
+                           hipStream_t stream) {
   return launch_k(false, tile_map_kernel, dim3(1), dim3(1024), 0, stream, offs, E, M, max_row_tiles(M, E),
-                  max_rows, tt.table, tt.count, tt.split_cnt);
+                  max_rows, tile_table_in(ws, M, E), with_small ? max_small_tiles(M, E) : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -54,9 +52,10 @@ int gemm_fwd_tile_rows() { return kFwdTileRows; }
 
 static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// The tile plan: header, split-tile counters, tile table.
+// The tile plan: header, split-tile counters, tile table, small-tile table.
 size_t gemm_plan_bytes(int64_t M, int E) {
-  return sizeof(int4) + kSplitTiles * sizeof(int) + (size_t)max_row_tiles((int)M, E) * sizeof(int4) + 256;
+  return sizeof(int4) + kSplitTiles * sizeof(int) +
+         (size_t)(max_row_tiles((int)M, E) + max_small_tiles((int)M, E)) * sizeof(int4) + 256;
 }
 
 // Partial sums of the split leftover tiles: one piece per workgroup at most.
@@ -86,21 +85,56 @@ void probe_chain_arm(const hipEvent_t* events, int n_launches) {
   p.chain_n = n_launches > 0 ? n_launches : 0;
 }
 
+// Weight rows per tile if a forward GEMM over `cols` weight rows per expert
+// takes the small-tile kernel, 0 if the 320 x 256 kernel.
+//
+// Up to kSmallAvgRows rows per expert on average the GEMM streams weights
+// and the small tiles' deeper ring is ahead (Qwen3-30B-A3B experts, both
+// GEMMs and the K-way sum: 2 rows 243 -> 196 us, 21 rows 283 -> 230, 63
+// rows 299 -> 251, 96 rows 315 -> 281; DeepSeek-V3's 94 rows 632 -> 530); at
+// 125-128 rows many experts need a second 128-row tile and it is not (331 ->
+// 337 us, 664 -> 680 us).  With more rows per expert it pays where the large
+// tiles leave the chip idle in their last round: the rounds of each tiling
+// are weighed with its time per 64-k stage (measured on whole rounds:
+// 2.0 us for 320 x 256, 1.08 for 128 x 256, 0.66 for 128 x 128, 0.85 for
+// 64 x 256 and 0.5 for 64 x 128), e.g. 4 experts of 2048 x 1024 with 2000
+// rows 98 -> 57 us and 8000 rows 121 us against 133 (kept large), while two
+// or more rounds of large tiles are better left alone (Llama4-Scout, 128
+// rows per expert: 568 us against 664).
+static int small_tile_cols(int M, int E, int64_t cols) {
+  const int rows = small_tile_rows(M, E);
+  if (rows == 0) return 0;
+  const int64_t G = (num_cus() + 7) & ~7;
+  // token tiles of at most h rows: one per hit expert, or by the row count
+  // with a partial tile for every third expert
+  auto qtiles = [&](int h) {
+    const int64_t hit = std::min(E, M);
+    return std::max<int64_t>(hit, (M + h - 1) / h + (hit - 1) / 3);
+  };
+  auto tiles = [&](int h, int c) { return qtiles(h) * ((cols + c - 1) / c); };
+  auto cost = [&](int h, int c, int64_t stage) { return (tiles(h, c) + G - 1) / G * stage; };
+  const int64_t c128 = cost(rows, 128, rows == 64 ? 50 : 66), c256 = cost(rows, 256, rows == 64 ? 85 : 108);
+  const int small = c128 < c256 ? 128 : 256;
+  if (M <= kSmallAvgRows * (int64_t)E) return small;
+  return tiles(kFwdTileRows, 256) < 2 * G && std::min(c128, c256) < cost(kFwdTileRows, 256, 200) ? small : 0;
+}
+
 // plan: the tile plan; part: the partial-sum area of split leftover tiles
 // (nullable: no split).  table_ready: `plan` already holds the tile table
 // of these rows (built for kFwdTileRows-row tiles), so no tile-map launch.
 static hipError_t fwd(int epi, FwdGemm g, const int* offs, int E, int M, void* plan, float* part,
                       hipStream_t stream, bool table_ready = false) {
   if (!table_ready) {
-    hipError_t err = launch_tile_map(offs, E, M, kFwdTileRows, plan, stream);
+    hipError_t err = launch_tile_map(offs, E, M, kFwdTileRows, plan, true, stream);
     if (err != hipSuccess) return err;
   }
-  const TileTable tt = tile_table_in(plan);
-  g.table = tt.table;
-  g.n_qtiles = tt.count;
+  const TileTable tt = tile_table_in(plan, M, E);
+  const int small = small_tile_cols(M, E, epi == EPI_SWIGLU ? 2 * (int64_t)g.n : g.n);
+  g.table = small ? tt.small_table : tt.table;
+  g.n_qtiles = small ? tt.small_count : tt.count;
   g.split_cnt = tt.split_cnt;
   g.part = part;
-  return launch_fwd_gemm(epi, g, stream);
+  return launch_fwd_gemm(epi, g, tt.small_rows, small, stream);
 }
 static hipError_t fwd(int epi, FwdGemm g, const int* offs, int E, int M, void* ws, hipStream_t stream) {
   return fwd(epi, g, offs, E, M, ws, split_part_in(ws, M, E), stream);
@@ -176,7 +210,7 @@ hipError_t launch_moe_experts_forward(const void* tokens, int T, int D, int H, i
   float* part = split_part_in(own_plan, M, E);
   if (tp == nullptr) {
     tp = own_plan;
-    if ((err = launch_tile_map(offs, E, M, kFwdTileRows, tp, stream)) != hipSuccess) return err;
+    if ((err = launch_tile_map(offs, E, M, kFwdTileRows, tp, true, stream)) != hipSuccess) return err;
   }
   if (permute_first) {
     err = launch_gather_rows(tokens, sorted_idx, score_before ? sorted_scores : nullptr, false, T, M, M, D, K,
@@ -205,9 +239,9 @@ hipError_t launch_moe_experts_forward(const void* tokens, int T, int D, int H, i
 // ---- fp8 forward (gemm_fp8.hip) ----------------------------------------------
 static hipError_t fp8(int epi, Fp8Args a, const int* offs, int E, int M, void* ws,
                       hipStream_t stream) {
-  hipError_t err = launch_tile_map(offs, E, M, kFp8TileRows, ws, stream);
+  hipError_t err = launch_tile_map(offs, E, M, kFp8TileRows, ws, false, stream);
   if (err != hipSuccess) return err;
-  const TileTable tt = tile_table_in(ws);
+  const TileTable tt = tile_table_in(ws, M, E);
   a.table = tt.table;
   a.n_qtiles = tt.count;
   return launch_fp8_gemm(epi, a, stream);
@@ -273,9 +307,9 @@ hipError_t launch_grouped_mm_fp8_unpermute(const void* aq, const float* sa, cons
 
 static hipError_t dgrad(int epi, DgradGemm g, const int* offs, int E, int M, void* plan, float* part,
                         hipStream_t stream) {
-  hipError_t err = launch_tile_map(offs, E, M, kFwdTileRows, plan, stream);
+  hipError_t err = launch_tile_map(offs, E, M, kFwdTileRows, plan, false, stream);
   if (err != hipSuccess) return err;
-  const TileTable tt = tile_table_in(plan);
+  const TileTable tt = tile_table_in(plan, M, E);
   g.table = tt.table;
   g.n_qtiles = tt.count;
   g.split_cnt = tt.split_cnt;
@@ -344,7 +378,7 @@ hipError_t launch_grouped_mm_wgrad(const void* dy, const void* x, const int* off
       const int avg_stages = (M / E + 63) / 64;
       while (np > 1 && avg_stages < np * kSplitMinStages) --np;
       if (np > 1) {
-        TileTable tt = tile_table_in(ws);
+        TileTable tt = tile_table_in(ws, M, E);
         hipError_t err = launch_split_cnt_zero(tt.split_cnt, rt, stream);
         if (err != hipSuccess) return err;
         a.part = split_part_in(ws, M, E);

@@ -34,24 +34,50 @@ __device__ __forceinline__ float clamp_nan(float x, float L) {
 constexpr int kTileRows = 128;
 constexpr int kFwdTileRows = 320;
 
-// Tile plan of a token-row GEMM: int4 header {number of tiles, ...}, the
-// arrival counters of the split tail tiles (kSplitTiles ints, zeroed
-// whenever a table is built and left at zero by every GEMM that uses them),
-// then the tile table.
+// Tile plan of a token-row GEMM: int4 header {number of tiles, number of
+// small tiles, ...}, the arrival counters of the split tail tiles
+// (kSplitTiles ints, zeroed whenever a table is built and left at zero by
+// every GEMM that uses them), the tile table, then (small_tile_rows(M, E) >
+// 0) the table of the small-tile kernel.
 constexpr int kSplitTiles = 512;
 struct TileTable {
   int* count;
   int* split_cnt;
   int4* table;
+  int small_rows;  // largest small tile, 0: no small table
+  int* small_count;
+  int4* small_table;
 };
 
 inline int max_row_tiles(int M, int E) { return M / kTileRows + E + 1; }
 
-inline TileTable tile_table_in(void* ws) {
+// Small-tile kernel (gemm_small.hip): token tiles of small_tile_rows(M, E)
+// rows at most, 128 or 256 weight rows.  Whether a GEMM of a plan takes it,
+// and with how many weight rows, is small_tile_cols' choice (gemm.hip); the
+// table exists wherever it could be chosen.  64-row tiles for experts that
+// mostly fit one, and for few rows in all (one expert of 7168 x 2048, 200
+// rows: 71 us against 94 with 128-row tiles; from ~1000 rows the 128-row
+// tiles are ahead, 42 against 50 us on 4 experts of 2048 x 1024).
+constexpr int kSmallAvgRows = 100;
+constexpr int kSmallMaxRows = 8192;
+inline int small_tile_rows(int M, int E) {
+  if (M <= 32 * (int64_t)E + 31 || M <= 768) return 64;
+  return M <= kSmallAvgRows * (int64_t)E || M <= kSmallMaxRows ? 128 : 0;
+}
+// An expert's c rows make at most ceil(c / rows) tiles.
+inline int max_small_tiles(int M, int E) {
+  const int rows = small_tile_rows(M, E);
+  return rows > 0 ? M / rows + E + 1 : 0;
+}
+
+inline TileTable tile_table_in(void* ws, int M, int E) {
   TileTable t;
   t.count = (int*)ws;
   t.split_cnt = (int*)ws + 4;
   t.table = (int4*)(t.split_cnt + kSplitTiles);
+  t.small_rows = small_tile_rows(M, E);
+  t.small_count = t.count + 1;
+  t.small_table = t.table + max_row_tiles(M, E);
   return t;
 }
 
@@ -71,20 +97,18 @@ constexpr int kSplitMaxPieces = 8;
 constexpr int kSplitMinStages = 8;
 constexpr int kSplitMaxRounds = 6;
 
-// Builds the tile table with one workgroup of NT threads (every thread
+// Builds one tile table with one workgroup of NT threads (every thread
 // calls it; it synchronises the workgroup).  `range(e, r0, r1)` gives the
 // rows [r0, r1) of expert e.  An expert's rows are split into the fewest
 // tiles of at most max_rows rows, of equal height rounded up to 32 rows
 // (540 rows at max_rows = 320 give 2 tiles of 288 rather than 320 + 220);
 // tiles are numbered in expert order.  Entries past the last tile, up to
-// max_tiles, are {-1, 0, 0, 0}.  The split-tile arrival counters are
-// zeroed.  sh: NT / 64 + 1 ints of LDS.
+// max_tiles, are {-1, 0, 0, 0}.  sh: NT / 64 + 1 ints of LDS.
 template <int NT, typename Range>
 __device__ void block_tile_table(Range range, int E, int max_tiles, int max_rows, int4* __restrict__ table,
-                                 int* __restrict__ count, int* __restrict__ split_cnt, int* sh) {
+                                 int* __restrict__ count, int* sh) {
   constexpr int NW = NT / kWave;
   const int tid = threadIdx.x;
-  for (int i = tid; i < kSplitTiles; i += NT) split_cnt[i] = 0;
   const int w = tid / kWave, l = lane_id();
   int carry = 0;
   for (int e0 = 0; e0 < E; e0 += NT) {
@@ -120,7 +144,17 @@ __device__ void block_tile_table(Range range, int E, int max_tiles, int max_rows
   if (tid == 0) *count = min(carry, max_tiles);
 }
 
-// Forward GEMM description (gemm_fwd.hip).
+// The whole plan: both tables (the small one where it exists) and zeroed
+// split-tile arrival counters.
+template <int NT, typename Range>
+__device__ void block_tile_plan(Range range, int E, int max_tiles, int max_rows, const TileTable& t,
+                                int max_small, int* sh) {
+  for (int i = threadIdx.x; i < kSplitTiles; i += NT) t.split_cnt[i] = 0;
+  block_tile_table<NT>(range, E, max_tiles, max_rows, t.table, t.count, sh);
+  if (max_small > 0) block_tile_table<NT>(range, E, max_small, t.small_rows, t.small_table, t.small_count, sh);
+}
+
+// Forward GEMM description (gemm_fwd.hip, gemm_small.hip).
 //   act [M][kred] bf16, w [E][N or 2N][kred] bf16.
 //   EPI_SWIGLU: n = H (w holds 2H rows: gate then up), out [M][H], h_out [M][2H].
 //   EPI_STORE / EPI_SCATTER: n = N, out [M or n_dest][N].
@@ -267,10 +301,14 @@ constexpr int kFp8TileRows = 256;
 
 int num_cus();
 
-hipError_t launch_tile_map(const int* offs, int E, int M, int max_rows, void* ws,
+// with_small: also the small-tile table, where small_tile_rows(M, E) > 0.
+hipError_t launch_tile_map(const int* offs, int E, int M, int max_rows, void* ws, bool with_small,
                            hipStream_t stream);
-// Forward GEMM over a tile table of at most kFwdTileRows rows per tile.
-hipError_t launch_fwd_gemm(int epi, const FwdGemm& g, hipStream_t stream);
+// Forward GEMM over a tile table of at most kFwdTileRows rows per tile
+// (small_cols == 0), or of at most small_rows rows and with small_cols
+// weight rows per tile (gemm_small.hip).
+hipError_t launch_fwd_gemm(int epi, const FwdGemm& g, int small_rows, int small_cols, hipStream_t stream);
+hipError_t launch_small_gemm(int epi, FwdArgs a, int tile_rows, int tile_cols, hipStream_t stream);
 // dgrad GEMM (EPI_STORE or EPI_SWIGLU_BWD) over the same tile table.
 hipError_t launch_dgrad_gemm(int epi, const DgradGemm& g, hipStream_t stream);
 // fp8 forward GEMM over a tile table of at most kFp8TileRows rows per tile.

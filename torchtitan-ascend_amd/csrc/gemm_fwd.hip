@@ -840,7 +840,7 @@ int num_cus() {
   return cus;
 }
 
-hipError_t launch_fwd_gemm(int epi, const FwdGemm& g, hipStream_t stream) {
+hipError_t launch_fwd_gemm(int epi, const FwdGemm& g, int small_rows, int small_cols, hipStream_t stream) {
   FwdArgs a = {};
   a.q = (const bf16_t*)g.act;
   a.ldq = g.kred;
@@ -865,6 +865,7 @@ hipError_t launch_fwd_gemm(int epi, const FwdGemm& g, hipStream_t stream) {
     a.limit = g.limit;
     a.h_out = (bf16_t*)g.h_out;
     a.ldh = 2 * (int64_t)g.n;
+    if (small_cols) return launch_small_gemm(epi, a, small_rows, small_cols, stream);
     if (a.q_index) return launch_fwd<EPI_SWIGLU, false, true>(a, stream);
     return launch_fwd<EPI_SWIGLU>(a, stream);
   }
@@ -877,6 +878,7 @@ hipError_t launch_fwd_gemm(int epi, const FwdGemm& g, hipStream_t stream) {
   a.n_dest = g.n_dest;
   a.accumulate = g.accumulate;
   a.scale_sigmoid = g.scale_sigmoid;
+  if (small_cols) return launch_small_gemm(epi, a, small_rows, small_cols, stream);
   if (epi == EPI_SCATTER) return launch_fwd<EPI_SCATTER>(a, stream);
   return launch_fwd<EPI_STORE>(a, stream);
 }

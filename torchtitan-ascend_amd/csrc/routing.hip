@@ -154,11 +154,10 @@ struct RouteExtras {
   int* counts;                // int32 [E]
   int* offsets;               // int32 [E + 1], exclusive
   float* tokens_per_expert;   // fp32 [E], += counts
-  int4* plan_table;           // tile table (gemm_common.h block_tile_table)
-  int* plan_count;
-  int* plan_split_cnt;
+  TileTable plan;             // tile plan (gemm_common.h block_tile_plan), null table: none
   int plan_max_tiles;
   int plan_max_rows;
+  int plan_max_small;
 };
 
 template <typename IdxT, bool FUSED>
@@ -305,13 +304,12 @@ __global__ __launch_bounds__(kRouteThreads) void route_rank_kernel(
       }
     }
     __syncthreads();
-    if (blockIdx.x == 0 && x.plan_table) {
+    if (blockIdx.x == 0 && x.plan.table) {
       auto range = [&](int e, int& r0, int& r1) {
         r0 = sh_start[e];
         r1 = sh_start[e + 1];
       };
-      block_tile_table<kRouteThreads>(range, E, x.plan_max_tiles, x.plan_max_rows, x.plan_table, x.plan_count,
-                                      x.plan_split_cnt, sh_scan);
+      block_tile_plan<kRouteThreads>(range, E, x.plan_max_tiles, x.plan_max_rows, x.plan, x.plan_max_small, sh_scan);
     }
   }
   // Running base of (wave w, bucket b) = chunk base + counts of earlier waves.
@@ -449,17 +447,15 @@ hipError_t launch_route_from_hist(const void* labels, bool is64, int M, int E, c
   x.offsets = offsets;
   x.tokens_per_expert = tokens_per_expert;
   if (plan) {
-    const TileTable tt = tile_table_in(plan);
-    x.plan_table = tt.table;
-    x.plan_count = tt.count;
-    x.plan_split_cnt = tt.split_cnt;
+    x.plan = tile_table_in(plan, M, E);
     x.plan_max_tiles = max_row_tiles(M, E);
     x.plan_max_rows = plan_max_rows;
+    x.plan_max_small = max_small_tiles(M, E);
   }
   if (M == 0) {  // nothing routed: zero counts / offsets, an empty tile table
     hipError_t err = launch_k(false, route_scan_kernel, dim3(1), dim3(kScanThreads),
                               (uint32_t)((E + 2) * sizeof(int)), stream, hist, 0, E, 1, 0, counts, offsets);
-    if (err == hipSuccess && plan) err = launch_tile_map(offsets + 1, E, 0, plan_max_rows, plan, stream);
+    if (err == hipSuccess && plan) err = launch_tile_map(offsets + 1, E, 0, plan_max_rows, plan, true, stream);
     return err;
   }
   if (route_fused_scan(M, E))
@@ -471,7 +467,7 @@ hipError_t launch_route_from_hist(const void* labels, bool is64, int M, int E, c
                             stream, hist, (E + 1) * nchunks, E, nchunks, M, counts, offsets);
   if (err == hipSuccess) err = launch_rank<false>(labels, is64, scores, M, E, nchunks, hist, sorted_idx, inverse,
                                       sorted_scores, RouteExtras{}, stream);
-  if (err == hipSuccess && plan) err = launch_tile_map(offsets + 1, E, M, plan_max_rows, plan, stream);
+  if (err == hipSuccess && plan) err = launch_tile_map(offsets + 1, E, M, plan_max_rows, plan, true, stream);
   if (err == hipSuccess && tokens_per_expert) {
     err = launch_k(false, accumulate_counts_kernel, dim3((E + 255) / 256), dim3(256), 0, stream, counts, E,
                    tokens_per_expert);
