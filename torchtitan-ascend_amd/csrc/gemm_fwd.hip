@@ -9,27 +9,35 @@
 //
 // Tile: up to 320 token rows (Q) x 256 weight rows (P); k in stages of 64.
 //   * 8 waves, two per SIMD, in a 2 x 4 arrangement: wave (wq, wp) owns 64
-//     weight rows and the tile's 32-row token blocks wq, wq + 2, ... (up to
-//     5 of them, 2 x 5 accumulators of v_mfma_f32_32x32x16_bf16, 160 fp32
+//     weight rows and 16 rows of each of the tile's 32-row token blocks (up
+//     to 10; 4 x 10 accumulators of v_mfma_f32_16x16x32_bf16, 160 fp32
 //     registers per lane).  The block count follows the tile's height (the
 //     k loop is instantiated per count), so a 256-row tile costs 256 rows of
 //     MFMA, LDS reads and token-row DMA, not 320.  The MFMA A operand is the
 //     weight tile, B the token tile, so a lane holds 4 consecutive output
-//     columns per register group.  SWIGLU: a wave's weight rows are 32 gate
-//     rows and the 32 matching up rows.
+//     columns per block.  SWIGLU: a wave's weight rows are 32 gate rows and
+//     the 32 matching up rows.
 //   * Two LDS stage buffers of 72 KB (32 KB weights + 40 KB tokens, rows of
 //     128 bytes = one full cache line per row and stage) filled by
 //     global_load_lds_dwordx4 (HBM/L2 -> LDS without VGPR staging).  A DMA
 //     instruction moves 8 whole rows; half-line rows (k stages of 32) cost
 //     twice the L2 requests per byte and capped the load rate.  The 16-byte
-//     chunk c of row r sits at c ^ ((r ^ (r >> 3)) & 7): the 8 (and 16)
-//     consecutive rows a fragment read serves per LDS cycle hit distinct
-//     banks.  A wave's DMA writes 1 KB of LDS contiguously, so the
-//     permutation is applied to the global addresses.
-//   * MFMA fragments are read one k16 step ahead; the single barrier of a
-//     stage sits before its last k16 step, after the last reads of the stage,
-//     and is where the next-but-one stage's weight rows are issued into the
-//     freed buffer; its token rows follow one k16 step later.
+//     chunk c of row r sits at c ^ ((r ^ (r >> 3)) & 7), which keeps the
+//     fragment reads free of bank conflicts.  A wave's DMA writes 1 KB of LDS
+//     contiguously, so the permutation is applied to the global addresses.
+//   * A stage is worked off token block by token block, with all of its
+//     weight fragments in registers.  Its weight rows and first token blocks
+//     are therefore free early, and the next-but-one stage's DMAs into them
+//     are in flight for almost two stages; they go out one at a time between
+//     the MFMAs (run_tile).
+//   * What bounds it: at C3 w13 the k loop runs at 1.65-1.95 GHz (the chip
+//     lowers its clock under MFMA load) with the matrix cores ~73 % busy, the
+//     rest of a stage lost around its two barriers; without the DMAs the
+//     same loop holds 2.2 GHz.  Measured, one box, against 32x32x16 MFMAs
+//     over k16 steps with each stage's DMAs issued in two bursts: C2 w13 401
+//     -> 381 us, w2 245 -> 235, dgrad + SwiGLU backward 344 -> 279; C3 w13
+//     1257 -> 1183, w2 676 -> 633, dgrad + SwiGLU backward 768 -> 699, dgrad
+//     1326 -> 1267; C4 w13 1642 -> 1549, w2 904 -> 850 us.
 //   * Per tile, a wave-uniform byte base (SGPRs) plus one 32-bit per-lane
 //     offset per DMA instruction; per stage only the k offset changes.
 //   * Persistent: one workgroup per CU walks the tile list with stride
@@ -69,8 +77,8 @@ constexpr int TQ = kFwdTileRows;  // 320 token rows
 constexpr int TP = 256;           // weight rows
 constexpr int WAVES = 8;          // 2 per SIMD
 constexpr int WPN = WAVES / 2;    // waves along the weight rows (2 along the token rows)
-constexpr int NJ = TQ / 64;       // 32-row token blocks per wave
-constexpr int NPB = TP / 32 / WPN;  // 32-row weight blocks per wave
+constexpr int NJ = TQ / 32;       // 16-row token blocks per wave
+constexpr int NPB = TP / 16 / WPN;  // 16-row weight blocks per wave
 constexpr int TK = 64;            // k per stage: 128-byte rows
 constexpr int NSTAGE = 2;
 constexpr int FTHREADS = 64 * WAVES;
@@ -80,38 +88,43 @@ constexpr int STAGE_BYTES = P_BYTES + TQ * ROW_BYTES;  // 72 KB
 constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES;        // 144 KB
 constexpr int DMA_P = TP / 8 / WAVES;                  // 4 weight-row instructions per wave
 constexpr int DMA_Q = TQ / 8 / WAVES;                  // 5 token-row instructions per wave
-constexpr int DMA_PER_STAGE = DMA_P + DMA_Q;           // 9 per lane
-static_assert(TQ % 64 == 0 && TP == 256 && TQ % (8 * WAVES) == 0 && NPB % 2 == 0, "tile geometry");
+constexpr int QA = 2;  // token-row instructions issued with a stage's weight rows
+static_assert(TQ % 64 == 0 && TP == 256 && TQ % (8 * WAVES) == 0 && NPB == 4, "tile geometry");
 // EPI_SCATTER row metadata (destination row, scale) of a tile, DMA'd with
 // the tile's first stage into one of three LDS slots (tile round % 3): the
 // slot of round r + 3 is written only after round r's epilogue.
 constexpr int META_BYTES = TQ * 8;
 // Gathered token rows (q_index): the tile's source-row ids, DMA'd one tile
-// ahead into one of two LDS slots (tile round % 2).
+// ahead into one of two LDS slots (tile round % 2), and the byte offsets of
+// the rows being issued, which every wave keeps for the rows it moves.
 constexpr int IDX_OFF = LDS_BYTES + 3 * META_BYTES;
 constexpr int IDX_BYTES = TQ * 4;
-constexpr int LDS_TOTAL = IDX_OFF + 2 * IDX_BYTES;  // 154 KB
+constexpr int GOFF_OFF = IDX_OFF + 2 * IDX_BYTES;
+constexpr int LDS_TOTAL = GOFF_OFF + IDX_BYTES;  // 155 KB
 // Split tail tiles: whether this workgroup's piece arrived last, in the
 // stage buffers (free by then) past the ring the partial sums stream through.
 constexpr int FLAG_OFF = 8 * 16 * 1024;
 static_assert(FLAG_OFF + 16 <= LDS_BYTES, "flag inside the stage buffers");
-static_assert(kSplitPartBytes == (size_t)WAVES * NJ * NPB * 16 * 64 * 4, "partial-sum area of a piece");
+static_assert(kSplitPartBytes == (size_t)WAVES * NJ * NPB * 4 * 64 * 4, "partial-sum area of a piece");
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 typedef __attribute__((address_space(1))) int gint_t;
 typedef __attribute__((address_space(1))) floatx4_t gfloatx4_t;
 
-// Chunk permutation of the 512-byte reduction-major weight rows (PT): the
-// 8 rows n0..n0+3, n0+8..n0+11 one transposed read touches land on four
-// distinct 64-byte bank groups, two rows each.
-__device__ __forceinline__ int ptswz(int n) { return 4 * ((n ^ (n >> 3)) & 3); }
+// Chunk permutation of the 512-byte reduction-major weight rows (PT): the 16
+// rows 16 g + 8 t + 4 h .. + 3 (g = 0..3) that one transposed read touches, 32
+// bytes each, land on eight distinct 32-byte bank groups, two rows each.
+__device__ __forceinline__ int ptswz(int n) { return 2 * ((n & 3) | ((n >> 2) & 4)); }
 
-// MFMA fragments of one k16 step: NPB weight blocks, NJ token blocks.
-struct Frag {
-  bf16x8_t a[NPB];
-  bf16x8_t b[NJ];
-};
+// f(integral_constant) for A, A + 1, ..., B - 1.
+template <int A, int B, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (A < B) {
+    f(std::integral_constant<int, A>{});
+    static_for<A + 1, B>(f);
+  }
+}
 
 // PT (dgrad): the weight operand is reduction-major, w[e][n][k] with the
 // reduction n as rows and the output index k contiguous.  Its stage is 64
@@ -217,8 +230,13 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
   static_assert(WAVES == 8, "row block 8 i + w has chunk permutation term w");
   const int rr0 = 8 * w + drow;
   const uint32_t lch16 = (uint32_t)(((l & 7) ^ ((drow ^ w) & 7)) * 16);
-  uint32_t d_ptoff[PT ? DMA_P : 1];
-  uint32_t d_gqoff[GATHER ? DMA_Q : 1];
+  // PT: rows 2 (WAVES i + w) and + 1, 32 chunks each.  The chunk permutation
+  // depends on i through bit 3 (i % 2), which is bit 7 of the byte offset
+  // (rows are a multiple of 256 bytes apart); otherwise instruction i moves
+  // the uniform base.
+  uint32_t d_ptoff = 0;
+  // GATHER: byte offsets of this wave's rows (instruction i, row l / 8) in LDS
+  int* const goff = (int*)(smem + GOFF_OFF) + w * (DMA_Q * 8);
   auto dma_tile = [&](int r) {
     const int tile = tile_at(r);
     const int qt = tile / a.np_tiles;
@@ -229,26 +247,24 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     d_qblk8 = 4 * ((ti.z - ti.y + 31) >> 5);
     d_qmax = qmax;
     if constexpr (PT) {
-#pragma unroll
-      for (int i = 0; i < DMA_P; ++i) {
-        // instruction i of wave w: rows 2 (WAVES i + w) and + 1, 32 chunks each
-        const int row = 2 * (WAVES * i + w) + (l >> 5);
-        const int lc = (l & 31) ^ ptswz(row);
-        const int col = min(pt * TP + 8 * lc, a.n_p - 8) - pt * TP;
-        d_ptoff[i] = (uint32_t)(row * ldp2 + col * 2);
-      }
+      const int row = 2 * w + (l >> 5);
+      // a tile with 128 valid columns (N % 128 == 0) reads those twice
+      const int lc = ((l & 31) ^ ptswz(row)) & (a.n_p - pt * TP >= TP ? 31 : 15);
+      d_ptoff = (uint32_t)(row * ldp2 + lc * 16);
     } else {
       d_pmax = a.n_p - 1 - pt * (EPI == EPI_SWIGLU ? 128 : TP);
     }
     if constexpr (GATHER) {
       // Gathered rows: tile row rr reads source row q_index[row] / q_div,
-      // whose id was DMA'd into LDS while the previous tile was issued.
+      // whose id was DMA'd into LDS while the previous tile was issued.  Lane
+      // 8 i + j works out row j of this wave's instruction i.
       const int* ids = (const int*)(smem + IDX_OFF + (r & 1) * IDX_BYTES);
-#pragma unroll
-      for (int i = 0; i < DMA_Q; ++i) {
-        const int src = min(max(ids[min(rr0 + 64 * i, qmax)] / a.q_div, 0), a.n_q_in - 1);
-        d_gqoff[i] = (uint32_t)(src * a.ldq * 2) + lch16;
+      if (l < DMA_Q * 8) {
+        const int row = min(64 * (l >> 3) + 8 * w + (l & 7), qmax);
+        const int src = min(max(ids[row] / a.q_div, 0), a.n_q_in - 1);
+        goff[l] = (int)((uint32_t)src * (uint32_t)(a.ldq * 2));
       }
+      lds_wait();
       if (r + 1 < nmy) load_ids(r + 1);
     }
     if constexpr (PT)
@@ -277,18 +293,20 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
   // of the next one is advanced here rather than divided out per call.
   // Past the end the last stage is issued again.
   int n_r = 0, n_ks = nfull > 0 ? 0 : pc_k0, n_kend = nfull > 0 ? ksteps : pc_k1, n_left = total;
-  auto issue_p = [&](int s) {
+  auto issue_prep = [&](int s) {
     const int r = n_r, ks = n_ks;
     if (r != d_r) dma_tile(r);
     d_spb = d_pbase + (PT ? (uint64_t)ks * TK * a.ldp * 2 : (uint64_t)ks * ROW_BYTES);
     d_sqb = d_qbase + (uint64_t)ks * ROW_BYTES;
     d_sst = lds0 + (uint32_t)((s & 1) * STAGE_BYTES) + w * 1024;
+  };
+  auto issue_p1 = [&](int i) {
     const uint32_t ldp2 = (uint32_t)a.ldp * 2u;
-#pragma unroll
-    for (int i = 0; i < DMA_P; ++i) {
+    {
       uint32_t voff;
       if constexpr (PT) {
-        voff = d_ptoff[i];
+        dma16(d_ptoff ^ (128u * (i & 1)), d_spb + (uint64_t)(uint32_t)(i * 2 * WAVES) * (uint64_t)(a.ldp * 2), d_sst + i * (WAVES * 1024));
+        return;
       } else if constexpr (EPI == EPI_SWIGLU) {
         // rows 0..127 gate, 128..255 up: tile row rr is weight row pt * 128 +
         // (rr & 127), of the up half (hidden + ...) for rr >= 128
@@ -299,6 +317,8 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
       }
       dma16(voff, d_spb, d_sst + i * (WAVES * 1024));
     }
+  };
+  auto issue_advance = [&]() {
     // Advance to the next stage only now: whatever sits between the stage
     // barrier and these DMAs delays every stage (the empty asm keeps the
     // compiler from hoisting the update above them).  Selects, no branches.
@@ -316,81 +336,89 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     n_ks = wrap ? (full ? 0 : pc_k0) : nk;
     n_kend = wrap ? (full ? ksteps : pc_k1) : n_kend;
   };
-  // Token rows past the tile's last 32-row block are never read: skip
-  // their DMA (wave-uniform: instruction i moves row block WAVES * i + w).
-  auto issue_q = [&]() {
-    const uint32_t ldq2 = (uint32_t)a.ldq * 2u;
-#pragma unroll
-    for (int i = 0; i < DMA_Q; ++i) {
-      if (WAVES * i + w < d_qblk8) {
-        const uint32_t voff = GATHER ? d_gqoff[GATHER ? i : 0] : (uint32_t)min(rr0 + 64 * i, d_qmax) * ldq2 + lch16;
-        dma16(voff, d_sqb, d_sst + P_BYTES + i * (WAVES * 1024));
-      }
-    }
+  // Token rows: instruction i moves the tile's rows 64 i .. + 63.  The first
+  // QA always go out (rows past the tile repeat its last row), so the DMAs in
+  // flight at a stage barrier can be counted; past the tile's last 32-row
+  // block the others are skipped (wave-uniform: instruction i moves row block
+  // WAVES * i + w).
+  auto issue_q1 = [&](int i) {
+    const uint32_t voff = (GATHER ? (uint32_t)goff[8 * i + drow]
+                                  : (uint32_t)min(rr0 + 64 * i, d_qmax) * ((uint32_t)a.ldq * 2u)) + lch16;
+    const uint32_t dst = d_sst + P_BYTES + i * (WAVES * 1024);
+    if (i < QA)
+      dma16(voff, d_sqb, dst);
+    else
+      { if (WAVES * i + w < d_qblk8) dma16(voff, d_sqb, dst); }
   };
-  auto issue = [&](int s) {
-    issue_p(s);
-    issue_q();
+  auto issue_all = [&](int st) {
+    issue_prep(st);
+#pragma unroll
+    for (int i = 0; i < DMA_P; ++i) issue_p1(i);
+#pragma unroll
+    for (int i = 0; i < DMA_Q; ++i) issue_q1(i);
+    issue_advance();
   };
 
   // ---- fragment geometry -------------------------------------------------------
-  // Row 32m + r32 has cswz = fa ^ 4 * (m & 1) with fa = cswz(r32); all
-  // fragment blocks start at multiples of 32 rows.
-  const int r32 = l & 31;
-  const int half = l >> 5;
-  const int fa = cswz(r32);
-  // SWIGLU: blocks pb < NPB/2 are gate rows, pb + NPB/2 the matching up rows.
-  int arow[NPB];
+  // v_mfma_f32_16x16x32_bf16: lane l holds row l % 16 of a 16-row block and 8
+  // consecutive k, chosen by l / 16.  The four chunks of a stage's step t are
+  // t, 2 + t, 4 + t and 6 + t, the same for both operands: with neighbouring
+  // chunks (4 t + l / 16) the reads of 16 rows meet on the same LDS banks
+  // (measured 300 B/ns per CU against 555, as the 32-row reads).
+  // (The 32x32x16 form moves twice the accumulators per flop and, at the
+  // chip's power limit, runs at a lower clock: the k loop alone on random
+  // operands 1565 TFLOP/s against 1750.)
+  const int r16 = l & 15;
+  const int g4 = l >> 4;
+  const int fa = cswz(r16);
+  // First row of weight block pb of the wave.  SWIGLU: blocks 0, 1 are gate
+  // rows, 2, 3 the matching up rows.
+  const int arow0 = (EPI == EPI_SWIGLU ? 32 : 64) * wp;
+  auto arow = [&](int pb) { return arow0 + (EPI == EPI_SWIGLU ? 16 * (pb & 1) + 128 * (pb >> 1) : 16 * pb); };
+  // Fragment addresses: the chunk permutation cswz(row) & 7 of row 16 m + r16
+  // is fa ^ 2 m, so k32 step, weight block and token block are compile-time
+  // bits XORed into one lane register per operand, rebased per stage (held
+  // per chunk and buffer the addresses would not fit beside the accumulators).
+  const int lane_p = PT ? 0 : (arow0 + r16) * ROW_BYTES + (((2 * g4) ^ fa ^ ((arow0 >> 3) & 7)) << 4);
+  const int lane_q = P_BYTES + (16 * wq + r16) * ROW_BYTES + (((2 * g4) ^ fa ^ (2 * wq)) << 4);
+  // PT: lane l of 16-lane group g4 loads row 16 g4 + 8 t + 4 h + (l & 15) / 4
+  // (h = 0, 1: the two halves of its 8 reduction values), columns
+  // arow(pb) + 4 (l & 3) .. + 3; t and h do not enter ptswz of that row.
+  const int tr_row = 16 * g4 + ((l & 15) >> 2);
+  const int tr_base = tr_row * (TP * 2) + ((l & 1) << 3);
+  const int tr_chunk = ((l & 2) >> 1) ^ ptswz(tr_row) ^ (8 * wp);  // arow0 = 64 wp: 8 chunks
+  auto stage_base = [&](int lane, int s) {
+    int v = lane;
+    asm volatile("" : "+v"(v));  // (kept from being expanded outside the stage)
+    return v + (s & 1) * STAGE_BYTES;
+  };
+  // Weight fragments of k32 step t.
+  auto read_p = [&](bf16x8_t (&f)[NPB], int s, int t) {
+    if constexpr (PT) {
+      const int tb = stage_base(tr_base, s);
 #pragma unroll
-  for (int pb = 0; pb < NPB; ++pb)
-    arow[pb] = (EPI == EPI_SWIGLU)
-                   ? (pb < NPB / 2 ? (128 / WPN) * wp + 32 * pb : 128 + (128 / WPN) * wp + 32 * (pb - NPB / 2))
-                   : (TP / WPN) * wp + 32 * pb;
-  // PT: lane l of 16-lane group g = (l >> 4) & 3 loads row
-  // 16 kk + 8 (g >> 1) + 4 t + (l & 15) / 4, columns arow + 16 (g & 1) +
-  // 4 (l & 3) .. + 3 (t = 0, 1: the two halves of its 8 reduction values).
-  // With n = 16 kk + tr_row + 4 t, ptswz(n) = 4 (bsw ^ 2 (kk & 1)) for a
-  // per-lane bsw, so each (block, kk parity) has one per-lane chunk offset
-  // and kk, t only move the row by constants.
-  const int tr_row = 8 * ((l >> 5) & 1) + ((l & 15) >> 2);
-  const int tr_col = 16 * ((l >> 4) & 1) + 4 * (l & 3);
-  const int bsw = ((l >> 2) & 3) ^ ((l >> 5) & 1);
-  int trx[PT ? NPB : 1][2];
-  if constexpr (PT) {
-#pragma unroll
-    for (int pb = 0; pb < NPB; ++pb)
-#pragma unroll
-      for (int par = 0; par < 2; ++par)
-        trx[pb][par] = tr_row * (TP * 2) + ((tr_col & 4) << 1) +
-                       ((((arow[pb] + tr_col) >> 3) ^ (4 * (bsw ^ (2 * par)))) << 4);
-  }
-  // Token block j of wave wq is the tile's 32-row block m = 2j + wq, so the
-  // chunk permutation term 4 * (m & 1) is 4 * wq for every block of a wave.
-  // njv (an integral constant) is the wave's block count in this tile.
-  auto read_frag = [&](Frag& f, int s, int kk, auto njv) {
-    constexpr int NJV = decltype(njv)::value;
-    if constexpr (NJV == 0) return;
-    const char* st = smem + (s & 1) * STAGE_BYTES;
-#pragma unroll
-    for (int pb = 0; pb < NPB; ++pb) {
-      if constexpr (PT) {
+      for (int pb = 0; pb < NPB; ++pb) {
+        const int off = tb + ((tr_chunk ^ (2 * pb)) << 4);
         short4_t v[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int off = trx[pb][kk & 1] + (16 * kk + 4 * t) * (TP * 2);
-          v[t] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(st + off));
-        }
-        f.a[pb] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7));
-        continue;
+        for (int h = 0; h < 2; ++h)
+          v[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + off + (8 * t + 4 * h) * (TP * 2)));
+        f[pb] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7));
       }
-      const int pc = (2 * kk + half) ^ fa ^ (4 * ((arow[pb] >> 5) & 1));
-      f.a[pb] = *(const bf16x8_t*)(st + (arow[pb] + r32) * ROW_BYTES + pc * 16);
-    }
+    } else {
+      const int base = stage_base(lane_p, s);
 #pragma unroll
-    for (int j = 0; j < NJV; ++j) {
-      const int pc = (2 * kk + half) ^ fa ^ (4 * wq);
-      f.b[j] = *(const bf16x8_t*)(st + P_BYTES + (64 * j + 32 * wq + r32) * ROW_BYTES + pc * 16);
+      for (int pb = 0; pb < NPB; ++pb) {
+        const int m = EPI == EPI_SWIGLU ? pb & 1 : pb;  // 16-row step inside the wave's rows
+        f[pb] = *(const bf16x8_t*)(smem + (base ^ (t << 4) ^ ((2 * m) << 4)) + (arow(pb) - arow0) * ROW_BYTES);
+      }
     }
+  };
+  // Token fragments of the wave's block j (tile rows 32 j + 16 wq .. + 15).
+  auto read_q = [&](bf16x8_t (&f)[2], int base, int j) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      f[t] = *(const bf16x8_t*)(smem + (base ^ (t << 4) ^ ((4 * (j & 1)) << 4)) + j * 32 * ROW_BYTES);
   };
 
   // ---- prologue: stages 0 and 1 in flight, stage 0 landed -----------------------
@@ -400,67 +428,105 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     load_ids(0);
     wait_vm_barrier<0>();
   }
-  issue(0);
-  issue(1);
-  wait_vm_barrier<0>();
+  issue_all(0);
+  issue_all(1);
+  wait_vm_barrier<DMA_P + QA>();
 
   int s = 0;
   // nks: the unit's k stages (ksteps for a whole tile); piece: the unit is
   // a piece of a split leftover tile.
   auto run_tile = [&](auto njv, int r, int row0, int row1, int pt, int nks, bool piece) {
     constexpr int NJV = decltype(njv)::value;
-    Frag f0, f1;  // per tile: the first fragments are read at the tile's start
-    read_frag(f0, s, 0, njv);
-    constexpr int NJA = NJV > 0 ? NJV : 1;
-    floatx16_t acc[NPB][NJA];
+    constexpr int NU = NJV;
+    floatx4_t acc[NPB][NJV];
 #pragma unroll
     for (int i = 0; i < NPB; ++i)
 #pragma unroll
-      for (int j = 0; j < NJA; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-    auto mfma = [&](const Frag& f) {
-#pragma unroll
-      for (int j = 0; j < NJV; ++j)
-#pragma unroll
-        for (int pb = 0; pb < NPB; ++pb)
-          acc[pb][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[pb], f.b[j], acc[pb][j], 0, 0, 0);
+      for (int j = 0; j < NJV; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    // One stage, token block by token block (a unit: 8 MFMAs).  The wave holds
+    // the stage's weight fragments (2 k32 steps) and reads the token
+    // fragments two units ahead.
+    //   A (before unit 2): every wave has read the stage's weight rows and
+    //     its first four token blocks (tile rows 0..127), so the
+    //     next-but-one stage's weight rows and first QA token-row
+    //     instructions go into their place, spread over the following units
+    //     (a burst of all of them stalls every wave's MFMAs behind the CU's
+    //     address unit): they are in flight for almost two stages.
+    //   B (before the last two units): every wave has read the whole stage;
+    //     the rest of the next-but-one stage's token rows follow.  The wait
+    //     there is for the next stage, i.e. for all but the DMA_P + QA
+    //     instructions issued at A.
+    // The last two units run after B while the next stage's first fragments
+    // are read.
+    bf16x8_t fp[2][NPB], fq[3][2];
+    // DMA instruction d of the stage being issued: weight rows, then token rows
+    auto issue_d = [&](auto dc) {
+      constexpr int d = decltype(dc)::value;
+      if constexpr (d < DMA_P)
+        issue_p1(d);
+      else
+        issue_q1(d - DMA_P);
     };
-    // One stage: k16 steps 0..3, each computed from registers while the next
-    // is read.  Before step 3 every wave has read all of stage s; the barrier
-    // there also waits for stage s + 1 (the only stage in flight), and the
-    // weight rows of stage s + 2 are issued into stage s's buffer at once;
-    // its token rows follow one k16 step later, at the start of stage s + 1
-    // (both have landed by that stage's barrier).  A tile's last stage
-    // issues the whole next-but-one stage at its barrier, before the
-    // epilogue.  Every wave runs the same barrier sequence whatever its
-    // block count.
-    for (int ks = 0; ks + 1 < nks; ++ks, ++s) {
-      if (ks > 0) issue_q();
-      read_frag(f1, s, 1, njv);
-      mfma(f0);
-      read_frag(f0, s, 2, njv);
-      mfma(f1);
-      read_frag(f1, s, 3, njv);
-      mfma(f0);
-      wait_vm_barrier<0>();
-      issue_p(s + 2);
-      read_frag(f0, s + 1, 0, njv);
-      mfma(f1);
-    }
-    // Last stage of the tile: the next tile's first fragments are read at
-    // the start of that tile, with its block count.
-    if (nks > 1) issue_q();
-    read_frag(f1, s, 1, njv);
-    mfma(f0);
-    read_frag(f0, s, 2, njv);
-    mfma(f1);
-    read_frag(f1, s, 3, njv);
-    mfma(f0);
-    wait_vm_barrier<0>();
-    issue(s + 2);
-    mfma(f1);
-    ++s;
+    auto mfma_t = [&](int j, const bf16x8_t& q, int t) {
+#pragma unroll
+      for (int pb = 0; pb < NPB; ++pb)
+        acc[pb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp[t][pb], q, acc[pb][j], 0, 0, 0);
+    };
+#pragma unroll
+    for (int t = 0; t < 2; ++t) read_p(fp[t], s, t);
+    read_q(fq[0], stage_base(lane_q, s), 0);
+    if constexpr (NU > 1) read_q(fq[1], stage_base(lane_q, s), 1);
+    auto stage = [&](auto lastc) {
+      constexpr bool LAST = decltype(lastc)::value;
+      constexpr int NA = DMA_P + QA, ND = DMA_P + DMA_Q;
+      constexpr int UB = NU > 2 ? NU - 2 : 0, UA = UB < 2 ? UB : 2;
+      constexpr int SPAN = UB > UA ? UB - UA : 1;
+      bf16x8_t nq[2][2];
+      const int qb = stage_base(lane_q, s);
+      static_for<0, UB>([&](auto uc) {
+        constexpr int u = decltype(uc)::value;
+        if constexpr (u == UA) {
+          lds_barrier();
+          issue_prep(s + 2);
+        }
+        read_q(fq[(u + 2) % 3], qb, u + 2);
+        if constexpr (u >= UA) static_for<NA * (u - UA) / SPAN, NA * (u - UA + 1) / SPAN>(issue_d);
+        mfma_t(u, fq[u % 3][0], 0);
+        mfma_t(u, fq[u % 3][1], 1);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if constexpr (UA == UB) {
+        lds_barrier();
+        issue_prep(s + 2);
+        static_for<0, NA>(issue_d);
+      }
+      // the last units (one if the tile has one block), k32 step by step, so
+      // that the next stage's weight fragments can be read in between
+      wait_vm_barrier<NA>();
+      const int qbn = LAST ? 0 : stage_base(lane_q, s + 1);
+      static_for<0, 2>([&](auto tc) {
+        constexpr int t = decltype(tc)::value;
+        static_for<NA + (ND - NA) * t / 2, NA + (ND - NA) * (t + 1) / 2>(issue_d);
+        if constexpr (!LAST && t < NU) read_q(nq[t], qbn, t);
+        static_for<UB, NU>([&](auto uc) {
+          constexpr int u = decltype(uc)::value;
+          mfma_t(u, fq[u % 3][t], t);
+        });
+        if constexpr (!LAST) read_p(fp[t], s + 1, t);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      issue_advance();
+      if constexpr (!LAST) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          fq[0][i] = nq[0][i];
+          if constexpr (NU > 1) fq[1][i] = nq[1][i];
+        }
+      }
+      ++s;
+    };
+    for (int ks = 0; ks + 1 < nks; ++ks) stage(std::false_type{});
+    stage(std::true_type{});
 
     // ---- split leftover tile: publish this piece's sums; the last piece
     //      to arrive adds all of them in piece order (the same order
@@ -472,13 +538,12 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     if (__builtin_expect(piece, 0)) {  // (laid out away from the tile path)
       // Partial sums of leftover tile pc_t: np * kSplitPartBytes bytes at
       // part + pc_t * np * kSplitPartBytes, wave w's share (NPB * NJ blocks
-      // of 4 KB per piece) at w * np * NPB * NJ * 4 KB, laid out block-major,
-      // then piece, then the block's four 1 KB groups (lane l: 16 bytes at
-      // 16 l).  The last piece then reads one contiguous stream per wave:
-      // 1 KB chunk i is block i / (4 np), piece i / 4 % np, group i % 4.
+      // of 1 KB per piece) at w * np * NPB * NJ KB, laid out block-major, then
+      // piece (lane l: 16 bytes at 16 l).  The last piece then reads one
+      // contiguous stream per wave: 1 KB chunk i is block i / np, piece i % np.
       // The bases are made opaque here so that no address is computed (and
       // kept live) in the k loop.
-      constexpr uint32_t BLK = 4 * 1024;
+      constexpr uint32_t BLK = 1024;
       // (re-read here rather than held through the k loop)
       int info = pc_info;
       asm volatile("" : "+s"(info));
@@ -502,10 +567,7 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
 #pragma unroll
         for (int j = 0; j < NJV; ++j) {
           const uint64_t dst = pw + (uint64_t)((pb * NJV + j) * bstride + pc_j * BLK);
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            *(gfloatx4_t*)(dst + (uint32_t)(g * 1024) + loff) =
-                floatx4_t{acc[pb][j][4 * g], acc[pb][j][4 * g + 1], acc[pb][j][4 * g + 2], acc[pb][j][4 * g + 3]};
+          *(gfloatx4_t*)(dst + loff) = acc[pb][j];
         }
       wait_vm<0>();  // this wave's partial has reached L2
       __syncthreads();
@@ -532,15 +594,13 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
       // exactly one DMA is issued per chunk consumed (past the end: the last
       // chunk again, into the slot just read), so "at most 15 in flight"
       // means chunk i has landed.
-      if constexpr (NJV > 0) {
+      {
 #pragma unroll
         for (int pb = 0; pb < NPB; ++pb)
 #pragma unroll
-          for (int j = 0; j < NJV; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[pb][j][v] = 0.f;
+          for (int j = 0; j < NJV; ++j) acc[pb][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
         constexpr int RING = 16;
-        const int last = NPB * NJV * 4 * np - 1;
+        const int last = NPB * NJV * np - 1;
         const uint32_t ring = lds0 + (uint32_t)w * (RING * 1024);
         auto fetch = [&](int i) {
           dma16(loff, pw + (uint32_t)min(i, last) * 1024u, ring + (uint32_t)(i & (RING - 1)) * 1024u);
@@ -554,108 +614,109 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
 #pragma unroll
           for (int j = 0; j < NJV; ++j)
             for (int q = 0; q < np; ++q) {
-#pragma unroll
-              for (int g = 0; g < 4; ++g) {
-                wait_vm<RING - 1>();
-                const float4 v = *(const float4*)(rbase + (i & (RING - 1)) * 1024);
-                acc[pb][j][4 * g] += v.x;
-                acc[pb][j][4 * g + 1] += v.y;
-                acc[pb][j][4 * g + 2] += v.z;
-                acc[pb][j][4 * g + 3] += v.w;
-                fetch(i + RING);  // after the adds: the slot's read has completed
-                ++i;
-              }
+              wait_vm<RING - 1>();
+              acc[pb][j] += *(const floatx4_t*)(rbase + (i & (RING - 1)) * 1024);
+              fetch(i + RING);  // after the adds: the slot's read has completed
+              ++i;
             }
         wait_vm<0>();
       }
     }
 
-    // ---- epilogue: acc[pb][j][4g + i] is (token row 64j + 32wq + r32,
-    //      weight row arow[pb] + 8g + 4 * half + i).  Column validity is
-    //      wave-uniform (H % 64 == 0 and N % 128 == 0 are required), row
-    //      validity is per lane.  The scheduling barriers keep each block's
-    //      accumulator reads next to their use (no 256-register hoist).
-    //      The lane row is re-materialised here (opaque copy) so that the
-    //      compiler does not keep per-block row offsets live across the k
-    //      loop, where every register is taken.
-    int er32 = r32;
-    asm volatile("" : "+v"(er32));
-    int ehalf = half;  // likewise for the lane's column half (store addresses)
-    asm volatile("" : "+v"(ehalf));
-    // EPI_SWIGLU_BWD: saved pre-activation of token block jj
-    auto load_h = [&](int jj, int pb, uint2 (&dst)[4][2]) {
-      if constexpr (EPI == EPI_SWIGLU_BWD) {
-        const int gq = row0 + 64 * jj + 32 * wq + er32;
-        const int qrow = min(gq, row1 - 1);
+    // ---- epilogue: acc[pb][j][i] is (token row 32 j + 16 wq + r16, weight
+    //      row arow(pb) + 4 g4 + i).  Column validity is uniform over a block
+    //      (H % 64 == 0 and N % 128 == 0 are required), row validity is per
+    //      lane.  The scheduling barriers keep each block's accumulator reads
+    //      next to their use (no 256-register hoist).  The lane's row and
+    //      column group are re-materialised here (opaque copies) so that the
+    //      compiler does not keep per-block offsets live across the k loop,
+    //      where every register is taken.
+    int er16 = r16;
+    asm volatile("" : "+v"(er16));
+    int eg4 = g4;
+    asm volatile("" : "+v"(eg4));
+    // A lane holds 4 consecutive columns (4 g4 ..) of each block.  For a pair
+    // of neighbouring blocks (p, p + 1), v_permlane16_swap exchanges the odd
+    // 16-lane rows of the first with the even rows of the second: lanes of
+    // group g4 then hold columns 8 (g4 / 2) .. + 7 of block p + (g4 & 1), one
+    // 16-byte store each.
+    auto pair16 = [&](const uint32_t (&p0)[2], const uint32_t (&p1)[2]) {
+      uint32_t x[2], y[2];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int col = min(pt * TP + arow[pb], a.n_p - 32) + 8 * g + 4 * half;
+      for (int d = 0; d < 2; ++d) {
+        const auto sw = __builtin_amdgcn_permlane16_swap(p0[d], p1[d], false, false);
+        x[d] = sw[0];
+        y[d] = sw[1];
+      }
+      return u32x4_t{x[0], x[1], y[0], y[1]};
+    };
+    const int pcol = 16 * (eg4 & 1) + 8 * (eg4 >> 1);  // the lane's columns in a block pair
+    // EPI_SWIGLU_BWD: saved pre-activation of token block jj
+    auto load_h = [&](int jj, uint2 (&dst)[NPB][2]) {
+      if constexpr (EPI == EPI_SWIGLU_BWD) {
+        const int qrow = min(row0 + 32 * jj + 16 * wq + er16, row1 - 1);
+#pragma unroll
+        for (int pb = 0; pb < NPB; ++pb) {
+          const int col = min(pt * TP + arow(pb), a.n_p - 16) + 4 * eg4;
           const bf16_t* hrow = a.h_in + (int64_t)qrow * a.ldh + col;
-          dst[g][0] = *(const uint2*)hrow;
-          dst[g][1] = *(const uint2*)(hrow + a.hidden);
+          dst[pb][0] = *(const uint2*)hrow;
+          dst[pb][1] = *(const uint2*)(hrow + a.hidden);
         }
       }
     };
-    // EPI_SWIGLU_BWD: the h values of block (j, pb) are loaded one block
+    // EPI_SWIGLU_BWD: the h values of token block j are loaded one block
     // ahead, into the other half of hbuf (double buffer).
-    uint2 hbuf[2][4][2];
-    if constexpr (EPI == EPI_SWIGLU_BWD) load_h(0, 0, hbuf[0]);
+    uint2 hbuf[2][NPB][2];
+    if constexpr (EPI == EPI_SWIGLU_BWD) load_h(0, hbuf[0]);
 #pragma unroll
     for (int j = 0; j < NJV; ++j) {
-      const int gq = row0 + 64 * j + 32 * wq + er32;
+      const int trow = 32 * j + 16 * wq + er16;
+      const int gq = row0 + trow;
       const bool row_ok = gq < row1;
       if constexpr (EPI == EPI_SWIGLU) {
         const float L = a.limit;
         // The clamp (swiglu_limit) is wave-uniform: one code path each, so
         // that the unclamped SwiGLU carries no min / max / select per value.
-        // Per 32-column block: gate and up are rounded to bf16 two at a time
-        // (one two-wide conversion each; the bf16 pairs are what h_out
-        // stores), then the row's stores share one address and one branch.
+        // Gate and up are rounded to bf16 two at a time (one two-wide
+        // conversion each; the bf16 pairs are what h_out stores).
         auto swiglu_rows = [&](auto clampc) {
           constexpr bool CLAMP = decltype(clampc)::value;
+          uint32_t ap[2][2], gp[2][2], up[2][2];
 #pragma unroll
-          for (int pb = 0; pb < NPB / 2; ++pb) {
-            uint32_t ap[4][2], gp[4][2], up[4][2];
+          for (int pb = 0; pb < 2; ++pb) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
+            for (int i2 = 0; i2 < 2; ++i2) {
+              // h is materialised in bf16 by the reference; SwiGLU reads it.
+              gp[pb][i2] = pack_bf16x2(acc[pb][j][2 * i2], acc[pb][j][2 * i2 + 1]);
+              up[pb][i2] = pack_bf16x2(acc[pb + 2][j][2 * i2], acc[pb + 2][j][2 * i2 + 1]);
+              float av[2];
 #pragma unroll
-              for (int i2 = 0; i2 < 2; ++i2) {
-                // h is materialised in bf16 by the reference; SwiGLU reads it.
-                const int v = 4 * g + 2 * i2;
-                gp[g][i2] = pack_bf16x2(acc[pb][j][v], acc[pb][j][v + 1]);
-                up[g][i2] = pack_bf16x2(acc[pb + NPB / 2][j][v], acc[pb + NPB / 2][j][v + 1]);
-                float av[2];
-#pragma unroll
-                for (int h2 = 0; h2 < 2; ++h2) {
-                  float gc = __uint_as_float(h2 ? (gp[g][i2] & 0xffff0000u) : (gp[g][i2] << 16));
-                  float uc = __uint_as_float(h2 ? (up[g][i2] & 0xffff0000u) : (up[g][i2] << 16));
-                  if constexpr (CLAMP) {
-                    gc = clamp_max_nan(gc, L);
-                    uc = clamp_nan(uc, L);
-                  }
-                  av[h2] = silu_f(gc) * uc;
+              for (int h2 = 0; h2 < 2; ++h2) {
+                float gc = __uint_as_float(h2 ? (gp[pb][i2] & 0xffff0000u) : (gp[pb][i2] << 16));
+                float uc = __uint_as_float(h2 ? (up[pb][i2] & 0xffff0000u) : (up[pb][i2] << 16));
+                if constexpr (CLAMP) {
+                  gc = clamp_max_nan(gc, L);
+                  uc = clamp_nan(uc, L);
                 }
-                ap[g][i2] = pack_bf16x2(av[0], av[1]);
+                av[h2] = silu_f(gc) * uc;
               }
+              ap[pb][i2] = pack_bf16x2(av[0], av[1]);
             }
-            if (row_ok) {
-              const int col = pt * 128 + (128 / WPN) * wp + 32 * pb + 4 * half;
-              bf16_t* orow = a.out + (int64_t)gq * a.ldo + col;
-#pragma unroll
-              for (int g = 0; g < 4; ++g) *(uint2*)(orow + 8 * g) = make_uint2(ap[g][0], ap[g][1]);
-              if (a.h_out) {
-                bf16_t* hrow = a.h_out + (int64_t)gq * a.ldh + col;
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                  *(uint2*)(hrow + 8 * g) = make_uint2(gp[g][0], gp[g][1]);
-                  *(uint2*)(hrow + a.hidden + 8 * g) = make_uint2(up[g][0], up[g][1]);
-                }
-              }
-            }
-            __builtin_amdgcn_sched_barrier(0);
           }
+          const u32x4_t av4 = pair16(ap[0], ap[1]);
+          const int col = pt * 128 + 32 * wp + pcol;
+          if (row_ok) *(u32x4_t*)(a.out + (int64_t)gq * a.ldo + col) = av4;
+          if (a.h_out) {
+            const u32x4_t gv4 = pair16(gp[0], gp[1]), uv4 = pair16(up[0], up[1]);
+            if (row_ok) {
+              bf16_t* hrow = a.h_out + (int64_t)gq * a.ldh + col;
+              *(u32x4_t*)hrow = gv4;
+              *(u32x4_t*)(hrow + a.hidden) = uv4;
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
         };
-        if (pt * 128 + (128 / WPN) * wp < a.n_p) {
+        if (pt * 128 + 32 * wp < a.n_p) {
           if (a.limit == a.limit)
             swiglu_rows(std::true_type{});
           else
@@ -664,56 +725,62 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
       } else if constexpr (EPI == EPI_SWIGLU_BWD) {
         // acc = dA = g for output columns p of the activation; with the saved
         // bf16 pre-activation h = [gate | up]: dgate, dup (clamp masks from
-        // the bf16 h, as the reference's autograd sees them).  The 8 h values
-        // of a 32-column block are loaded before any is used.
+        // the bf16 h, as the reference's autograd sees them).
         // Without a clamp the limit is +inf: minimum / maximum against it are
         // exact no-ops (NaN included) and the masks are forced true, so the
         // value loop has no branch on the clamp.
         const bool noclamp = !(a.limit == a.limit);
         const float L = noclamp ? __builtin_inff() : a.limit;
+        if (j + 1 < NJV) load_h(j + 1, hbuf[(j + 1) & 1]);
+        const uint2 (&hv)[NPB][2] = hbuf[j & 1];
 #pragma unroll
-        for (int pb = 0; pb < NPB; ++pb) {
-          const int blk = j * NPB + pb;
-          if (blk + 1 < NJV * NPB) load_h((blk + 1) / NPB, (blk + 1) % NPB, hbuf[(blk + 1) & 1]);
-          const uint2 (&hv)[4][2] = hbuf[blk & 1];
-          if (pt * TP + arow[pb] < a.n_p && row_ok) {
-            const int col0 = pt * TP + arow[pb] + 4 * half;
-            bf16_t* drow = a.out + (int64_t)gq * a.ldo + col0;
+        for (int pp = 0; pp < NPB; pp += 2) {
+          uint32_t dgp[2][2], dup[2][2], avp[2][2];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const uint2 hg = hv[g][0];
-              const uint2 hu = hv[g][1];
-              const float gate[4] = {bf16_to_f32(hg.x & 0xffff), bf16_to_f32(hg.x >> 16),
-                                     bf16_to_f32(hg.y & 0xffff), bf16_to_f32(hg.y >> 16)};
-              const float up[4] = {bf16_to_f32(hu.x & 0xffff), bf16_to_f32(hu.x >> 16),
-                                   bf16_to_f32(hu.y & 0xffff), bf16_to_f32(hu.y >> 16)};
-              float dg[4], du[4], av[4];
+          for (int b2 = 0; b2 < 2; ++b2) {
+            const int pb = pp + b2;
+            const uint2 hg = hv[pb][0];
+            const uint2 hu = hv[pb][1];
+            const float gate[4] = {bf16_to_f32(hg.x & 0xffff), bf16_to_f32(hg.x >> 16), bf16_to_f32(hg.y & 0xffff),
+                                   bf16_to_f32(hg.y >> 16)};
+            const float up[4] = {bf16_to_f32(hu.x & 0xffff), bf16_to_f32(hu.x >> 16), bf16_to_f32(hu.y & 0xffff),
+                                 bf16_to_f32(hu.y >> 16)};
+            float dg[4], du[4], av[4];
 #pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const float gd = acc[pb][j][4 * g + i];
-                float gc = gate[i], uc = up[i];
-                // torch.clamp's backward: where(in range, grad, 0), so exactly
-                // zero where it clamped and where h is NaN
-                const bool kg = noclamp | (gc <= L);
-                const bool ku = noclamp | ((uc >= -L) & (uc <= L));
-                gc = clamp_max_nan(gc, L);
-                uc = clamp_nan(uc, L);
-                const float sig = sigmoid_f(gc);
-                const float sv = gc * sig;
-                const float ds = sig * (1.f + gc * (1.f - sig));
-                dg[i] = kg ? gd * uc * ds : 0.f;
-                du[i] = ku ? gd * sv : 0.f;
-                av[i] = sv * uc;
-              }
-              *(uint2*)(drow + 8 * g) = make_uint2(pack_bf16x2(dg[0], dg[1]), pack_bf16x2(dg[2], dg[3]));
-              *(uint2*)(drow + a.hidden + 8 * g) =
-                  make_uint2(pack_bf16x2(du[0], du[1]), pack_bf16x2(du[2], du[3]));
-              if (a.a_out) {
-                bf16_t* arow_p = a.a_out + (int64_t)gq * a.hidden + col0 + 8 * g;
-                *(uint2*)arow_p = make_uint2(pack_bf16x2(av[0], av[1]), pack_bf16x2(av[2], av[3]));
-              }
-              __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < 4; ++i) {
+              const float gd = acc[pb][j][i];
+              float gc = gate[i], uc = up[i];
+              // torch.clamp's backward: where(in range, grad, 0), so exactly
+              // zero where it clamped and where h is NaN
+              const bool kg = noclamp | (gc <= L);
+              const bool ku = noclamp | ((uc >= -L) & (uc <= L));
+              gc = clamp_max_nan(gc, L);
+              uc = clamp_nan(uc, L);
+              const float sig = sigmoid_f(gc);
+              const float sv = gc * sig;
+              const float ds = sig * (1.f + gc * (1.f - sig));
+              dg[i] = kg ? gd * uc * ds : 0.f;
+              du[i] = ku ? gd * sv : 0.f;
+              av[i] = sv * uc;
             }
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+              dgp[b2][d] = pack_bf16x2(dg[2 * d], dg[2 * d + 1]);
+              dup[b2][d] = pack_bf16x2(du[2 * d], du[2 * d + 1]);
+              avp[b2][d] = pack_bf16x2(av[2 * d], av[2 * d + 1]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          const u32x4_t dg4 = pair16(dgp[0], dgp[1]), du4 = pair16(dup[0], dup[1]);
+          const int col0 = pt * TP + arow(pp) + pcol;
+          if (pt * TP + arow(pp) < a.n_p && row_ok) {
+            bf16_t* drow = a.out + (int64_t)gq * a.ldo + col0;
+            *(u32x4_t*)drow = dg4;
+            *(u32x4_t*)(drow + a.hidden) = du4;
+          }
+          if (a.a_out) {
+            const u32x4_t av4 = pair16(avp[0], avp[1]);
+            if (pt * TP + arow(pp) < a.n_p && row_ok) *(u32x4_t*)(a.a_out + (int64_t)gq * a.hidden + col0) = av4;
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -722,57 +789,37 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
         int orow_idx = gq;
         if constexpr (EPI == EPI_SCATTER) {
           const int* meta = (const int*)(smem + LDS_BYTES + (r % 3) * META_BYTES);
-          const int qrow = 64 * j + 32 * wq + er32;
-          if (a.dest) orow_idx = min(max(meta[qrow], 0), a.n_dest - 1);
+          if (a.dest) orow_idx = min(max(meta[trow], 0), a.n_dest - 1);
           if (a.row_scale) {
-            sc = __int_as_float(meta[TQ + qrow]);
+            sc = __int_as_float(meta[TQ + trow]);
             if (a.scale_sigmoid) sc = sigmoid_f(sc);
           }
         }
         bf16_t* orow = a.out + (int64_t)orow_idx * a.ldo;
 #pragma unroll
-        for (int pb = 0; pb < NPB; ++pb) {
-          if (pt * TP + arow[pb] < a.n_p) {
-            const floatx16_t& v = acc[pb][j];
-            uint32_t pk[4][2];
+        for (int pp = 0; pp < NPB; pp += 2) {
+          if (pt * TP + arow(pp) < a.n_p) {
+            uint32_t pk[2][2];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              pk[g][0] = pack_bf16x2(v[4 * g] * sc, v[4 * g + 1] * sc);
-              pk[g][1] = pack_bf16x2(v[4 * g + 2] * sc, v[4 * g + 3] * sc);
+            for (int b2 = 0; b2 < 2; ++b2) {
+              const floatx4_t& v = acc[pp + b2][j];
+              pk[b2][0] = pack_bf16x2(v[0] * sc, v[1] * sc);
+              pk[b2][1] = pack_bf16x2(v[2] * sc, v[3] * sc);
             }
-            // Lanes l and l ^ 32 hold the same output row, half h holding
-            // columns 8g + 4h .. + 3 of group g.  Swapping one group each
-            // way leaves lane half h with columns 16c + 8h .. + 7 (c = 0, 1),
-            // so every store is 16 bytes and 32 contiguous bytes per row.
-            // v_permlane32_swap(x, y) exchanges x of lanes 32..63 with y of
-            // lanes 0..31: with x = group 2c and y = group 2c + 1, the low
-            // half ends with {own 2c, partner's 2c} (columns 16c .. + 7) and
-            // the high half with {partner's 2c + 1, own 2c + 1}
-            // (columns 16c + 8 .. + 15), both in (x, y) order.
+            const u32x4_t val = pair16(pk[0], pk[1]);
+            const int col = pt * TP + arow(pp) + pcol;
+            if (row_ok) {
+              if (a.accumulate) {
+                // add to the row already there (bf16 + bf16, one rounding)
+                const u32x4_t prev = *(const u32x4_t*)(orow + col);
+                u32x4_t sum;
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-              uint32_t x[2], y[2];
-#pragma unroll
-              for (int d = 0; d < 2; ++d) {
-                const auto sw = __builtin_amdgcn_permlane32_swap(pk[2 * c][d], pk[2 * c + 1][d], false, false);
-                x[d] = sw[0];
-                y[d] = sw[1];
-              }
-              const u32x4_t val = u32x4_t{x[0], x[1], y[0], y[1]};
-              const int col = pt * TP + arow[pb] + 16 * c + 8 * ehalf;
-              if (row_ok) {
-                if (a.accumulate) {
-                  // add to the row already there (bf16 + bf16, one rounding)
-                  const u32x4_t prev = *(const u32x4_t*)(orow + col);
-                  u32x4_t sum;
-#pragma unroll
-                  for (int d = 0; d < 4; ++d)
-                    sum[d] = pack_bf16x2(bf16_to_f32(val[d] & 0xffffu) + bf16_to_f32(prev[d] & 0xffffu),
-                                         bf16_to_f32(val[d] >> 16) + bf16_to_f32(prev[d] >> 16));
-                  *(u32x4_t*)(orow + col) = sum;
-                } else {
-                  *(u32x4_t*)(orow + col) = val;
-                }
+                for (int d = 0; d < 4; ++d)
+                  sum[d] = pack_bf16x2(bf16_to_f32(val[d] & 0xffffu) + bf16_to_f32(prev[d] & 0xffffu),
+                                       bf16_to_f32(val[d] >> 16) + bf16_to_f32(prev[d] >> 16));
+                *(u32x4_t*)(orow + col) = sum;
+              } else {
+                *(u32x4_t*)(orow + col) = val;
               }
             }
           }
@@ -787,18 +834,22 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     const int qt = tile / a.np_tiles;
     const int pt = tile - qt * a.np_tiles;
     const int4 ti = sload_int4(a.table + qt);
-    // 32-row blocks of the tile (at most TQ / 32), interleaved over the two
-    // token-row waves: wave wq takes blocks wq, wq + 2, ...
-    const int nj = min((((ti.z - ti.y + 31) >> 5) + 1 - wq) >> 1, NJ);
+    // 32-row blocks of the tile (at most TQ / 32): each token-row wave takes
+    // 16 rows of every block
+    const int nj = min((ti.z - ti.y + 31) >> 5, NJ);
     const bool piece = r >= nfull;
     const int nks = piece ? pc_k1 - pc_k0 : ksteps;
     switch (nj) {
+      case 10: run_tile(std::integral_constant<int, 10>{}, r, ti.y, ti.z, pt, nks, piece); break;
+      case 9: run_tile(std::integral_constant<int, 9>{}, r, ti.y, ti.z, pt, nks, piece); break;
+      case 8: run_tile(std::integral_constant<int, 8>{}, r, ti.y, ti.z, pt, nks, piece); break;
+      case 7: run_tile(std::integral_constant<int, 7>{}, r, ti.y, ti.z, pt, nks, piece); break;
+      case 6: run_tile(std::integral_constant<int, 6>{}, r, ti.y, ti.z, pt, nks, piece); break;
       case 5: run_tile(std::integral_constant<int, 5>{}, r, ti.y, ti.z, pt, nks, piece); break;
       case 4: run_tile(std::integral_constant<int, 4>{}, r, ti.y, ti.z, pt, nks, piece); break;
       case 3: run_tile(std::integral_constant<int, 3>{}, r, ti.y, ti.z, pt, nks, piece); break;
       case 2: run_tile(std::integral_constant<int, 2>{}, r, ti.y, ti.z, pt, nks, piece); break;
-      case 1: run_tile(std::integral_constant<int, 1>{}, r, ti.y, ti.z, pt, nks, piece); break;
-      default: run_tile(std::integral_constant<int, 0>{}, r, ti.y, ti.z, pt, nks, piece); break;
+      default: run_tile(std::integral_constant<int, 1>{}, r, ti.y, ti.z, pt, nks, piece); break;
     }
   }
   wait_vm<0>();  // DMAs past the end have landed before the workgroup exits
