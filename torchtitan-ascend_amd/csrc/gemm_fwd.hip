@@ -347,8 +347,8 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     const uint32_t dst = d_sst + P_BYTES + i * (WAVES * 1024);
     if (i < QA)
       dma16(voff, d_sqb, dst);
-    else
-      { if (WAVES * i + w < d_qblk8) dma16(voff, d_sqb, dst); }
+    else if (WAVES * i + w < d_qblk8)
+      dma16(voff, d_sqb, dst);
   };
   auto issue_all = [&](int st) {
     issue_prep(st);

@@ -13,13 +13,22 @@
 //     output columns k (A operand, 4 consecutive k per lane and register
 //     group, so fp32 / bf16 results leave as 16- / 8-byte stores).
 //   * 8 waves (2 per SIMD), 2 (n) x 4 (k); each wave 128 n x 64 k =
-//     2 x 4 accumulators of v_mfma_f32_32x32x16_bf16.
+//     4 x 8 accumulators of v_mfma_f32_16x16x32_bf16 (half the accumulator
+//     traffic per flop of the 32x32x16 form and, at the chip's power limit,
+//     a ~12 % higher MFMA rate).
 //   * Stages of 64 rows m: x rows (64 x 512 bytes) and dy rows (64 x 512
 //     bytes) DMA'd by global_load_lds_dwordx4 into two 64 KB buffers, chunk
-//     c of row m stored at c ^ 4 ((m ^ (m >> 3)) & 3) (conflict-free
-//     transposed reads); one barrier per stage as in gemm_fwd.hip.
+//     c of row m stored at c ^ ptswz(m) (conflict-free transposed reads).
+//     As in gemm_fwd.hip a stage is worked off one 16-column dy block at a
+//     time with all of its x fragments in registers: its x rows are free
+//     early and the next-but-one stage's go out at once, one DMA between the
+//     MFMAs of each block; its dy rows follow at the stage's end.
+//     Measured against 32x32x16 MFMAs with both operands' DMAs in one burst
+//     per stage (one box, bf16 gradients): C3 routed dW13 1604 -> 1476 us,
+//     dW2 779 -> 726, shared dW13 1185 -> 1080, dW2 620 -> 564; C2 shapes
+//     dW13 530 -> 479, dW2 267 -> 246.
 //   * The last stage of an expert reads clamped rows past its end; their
-//     products are removed by zeroing those rows in the x fragments.
+//     products are removed by zeroing those rows in both operands' fragments.
 //   * Persistent over (expert, n tile, k tile), expert-major, the n tiles in
 //     strips of 4 with the k tile major inside a strip (see tile_of), with
 //     the XCD-aware slot mapping of gemm_fwd.hip; the DMA stream runs over
@@ -33,6 +42,8 @@
 //     piece writes its fp32 sums to the workspace and counts its arrival,
 //     and the last to arrive adds all of them in piece order (the same sum
 //     whichever arrives last) and runs the epilogue.
+#include <type_traits>
+
 #include "common.h"
 #include "dma_asm.h"
 #include "gemm_common.h"
@@ -48,8 +59,8 @@ constexpr int TP = 256;  // k per tile
 constexpr int TK = 64;   // rows m per stage
 constexpr int WAVES = 8;
 constexpr int WPN = 4;              // waves along k
-constexpr int NJ = TQ / 32 / 2;     // 4 n blocks per wave
-constexpr int NPB = TP / 32 / WPN;  // 2 k blocks per wave
+constexpr int NJ = TQ / 16 / 2;     // 8 n blocks of 16 per wave
+constexpr int NPB = TP / 16 / WPN;  // 4 k blocks of 16 per wave
 constexpr int THREADS = 64 * WAVES;
 constexpr int ROW_BYTES = 512;      // 256 bf16 columns of one row m
 constexpr int OP_BYTES = TK * ROW_BYTES;  // 32 KB per operand and stage
@@ -66,12 +77,17 @@ typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 typedef __attribute__((address_space(1))) int gint_t;
 typedef __attribute__((address_space(1))) floatx4_t gfloatx4_t;
 
-__device__ __forceinline__ int ptswz(int m) { return 4 * ((m ^ (m >> 3)) & 3); }
+// Chunk permutation of a row (as gemm_fwd.hip's reduction-major weights).
+__device__ __forceinline__ int ptswz(int m) { return 2 * ((m & 3) | ((m >> 2) & 4)); }
 
-struct Frag {
-  bf16x8_t a[NPB];  // x: k blocks
-  bf16x8_t b[NJ];   // dy: n blocks
-};
+// f(integral_constant) for A, A + 1, ..., B - 1.
+template <int A, int B, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (A < B) {
+    f(std::integral_constant<int, A>{});
+    static_for<A + 1, B>(f);
+  }
+}
 
 __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDmaArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -135,34 +151,42 @@ __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDma
 
   // ---- DMA stream: a cursor over (tile round, stage) --------------------------
   // instruction i of wave w moves rows 2 (WAVES i + w) and + 1 of an operand;
-  // lane l: row + (l >> 5), physical chunk l & 31.
+  // lane l: row + (l >> 5), physical chunk l & 31.  The chunk permutation
+  // depends on i through bit 3 (i % 2) only; a tile with 128 valid columns
+  // (N, K % 128 == 0) reads those twice.
   int c_r = 0, c_ks = 0;
   Tile c_t = tile_of(0);
-  auto issue = [&](int s) {
-    const int m_stage = c_t.m0 + TK * c_ks;
-    const int nvalid = c_t.m1 - m_stage;  // may be <= 0 for an expert without rows
-    const uint64_t xb = (uint64_t)(a.x + (int64_t)c_t.kt * TP);
-    const uint64_t yb = (uint64_t)(a.dy + (int64_t)c_t.nt * TQ);
-    const uint32_t st = lds0 + (uint32_t)((s & 1) * STAGE_BYTES) + w * 1024;
-    if (a.M > 0) {  // no rows at all: every stage is masked, nothing to load
-#pragma unroll
-    for (int i = 0; i < DMA_OP; ++i) {
-      const int row = 2 * (WAVES * i + w) + (l >> 5);
-      const int lc = (l & 31) ^ ptswz(row);
-      const int m = min(max(m_stage + min(row, nvalid - 1), 0), a.M - 1);
-      const int xcol = min(c_t.kt * TP + 8 * lc, a.K - 8) - c_t.kt * TP;
-      dma16((uint32_t)(m * a.ldx * 2 + xcol * 2), xb, st + i * (WAVES * 1024));
+  const int d_row = 2 * w + (l >> 5);
+  const int d_chunk = (l & 31) ^ ptswz(d_row);
+  uint64_t d_xb = 0, d_yb = 0;
+  int d_mstage = 0, d_last = 0, d_xmask = 31, d_ymask = 31;
+  uint32_t d_st = 0;
+  // bases of the stage issued next, into the buffer of stage s
+  auto issue_prep = [&](int s) {
+    d_mstage = c_t.m0 + TK * c_ks;
+    d_last = c_t.m1 - 1;  // below d_mstage for an expert without rows
+    d_xb = (uint64_t)(a.x + (int64_t)c_t.kt * TP);
+    d_yb = (uint64_t)(a.dy + (int64_t)c_t.nt * TQ);
+    d_xmask = a.K - c_t.kt * TP >= TP ? 31 : 15;
+    d_ymask = a.N - c_t.nt * TQ >= TQ ? 31 : 15;
+    if (a.M == 0) {  // no rows at all: every stage is masked; any readable address will do
+      d_xb = d_yb = (uint64_t)a.dw;
+      d_xmask = d_ymask = 15;
     }
-#pragma unroll
-    for (int i = 0; i < DMA_OP; ++i) {
-      const int row = 2 * (WAVES * i + w) + (l >> 5);
-      const int lc = (l & 31) ^ ptswz(row);
-      const int m = min(max(m_stage + min(row, nvalid - 1), 0), a.M - 1);
-      const int ycol = min(c_t.nt * TQ + 8 * lc, a.N - 8) - c_t.nt * TQ;
-      dma16((uint32_t)(m * a.lddy * 2 + ycol * 2), yb, st + OP_BYTES + i * (WAVES * 1024));
-    }
-    }
-    // advance; past the last stage keep re-loading it
+    d_st = lds0 + (uint32_t)((s & 1) * STAGE_BYTES) + w * 1024;
+  };
+  const int m_max = max(a.M - 1, 0);
+  auto row_of = [&](int i) { return min(max(min(d_mstage + d_row + 2 * WAVES * i, d_last), 0), m_max); };
+  auto issue_x = [&](int i) {
+    const uint32_t voff = (uint32_t)row_of(i) * (uint32_t)(a.ldx * 2) + (((d_chunk ^ (8 * (i & 1))) & d_xmask) << 4);
+    dma16(voff, d_xb, d_st + i * (WAVES * 1024));
+  };
+  auto issue_y = [&](int i) {
+    const uint32_t voff = (uint32_t)row_of(i) * (uint32_t)(a.lddy * 2) + (((d_chunk ^ (8 * (i & 1))) & d_ymask) << 4);
+    dma16(voff, d_yb, d_st + OP_BYTES + i * (WAVES * 1024));
+  };
+  // past the last stage keep re-loading it
+  auto issue_advance = [&]() {
     if (c_ks + 1 < c_t.nks) {
       ++c_ks;
     } else if (c_r + 1 < nmy) {
@@ -173,104 +197,139 @@ __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDma
   };
 
   // ---- fragments: transposed reads (see gemm_fwd.hip, PT) ---------------------
-  const int tr_row = 8 * ((l >> 5) & 1) + ((l & 15) >> 2);
-  const int tr_col = 16 * ((l >> 4) & 1) + 4 * (l & 3);
-  const int bsw = ((l >> 2) & 3) ^ ((l >> 5) & 1);
-  int arow[NPB], brow[NJ];
-#pragma unroll
-  for (int pb = 0; pb < NPB; ++pb) arow[pb] = (TP / WPN) * wp + 32 * pb;
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) brow[j] = (TQ / 2) * wq + 32 * j;
-  // Offset of the lane's 8-byte piece for a 32-column block at col0 (uniform)
-  // and reduction rows 16 kk + 4 t + tr_row: the chunk XOR depends on the
-  // lane and on kk & 1 only (see gemm_fwd.hip, PT).
-  const int tr_base = tr_row * ROW_BYTES + ((tr_col & 4) << 1);
-  const int tc8 = tr_col >> 3;
-  const int swz0 = 4 * bsw, swz1 = 4 * (bsw ^ 2);
-  auto tr8 = [&](const char* st, int col0, int kk) {
-    const int off = tr_base + ((((col0 >> 3) + tc8) ^ ((kk & 1) ? swz1 : swz0)) << 4) + (16 * kk) * ROW_BYTES;
-    short4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(st + off));
-    short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(st + off + 4 * ROW_BYTES));
+  // k32 step t: lane l of 16-lane group g4 holds rows 16 g4 + 8 t .. + 7 of
+  // column col0 + l % 16, from two reads of rows + 4 h + (l & 15) / 4,
+  // columns col0 + 4 (l & 3) .. + 3; t and h do not enter ptswz of the row.
+  const int r16 = l & 15;
+  const int g4 = l >> 4;
+  const int tr_row = 16 * g4 + (r16 >> 2);
+  // A block of 16 columns is two chunks: block m of the wave's columns and the
+  // permutation only XOR bits 5..8 of the lane's address.
+  const int tr_base = tr_row * ROW_BYTES + ((l & 1) << 3);
+  const int tr_chunk = ((l & 2) >> 1) ^ ptswz(tr_row);
+  const int arow0 = (TP / WPN) * wp, brow0 = (TQ / 2) * wq;
+  const int lane_x = tr_base + ((tr_chunk ^ (arow0 >> 3)) << 4);
+  const int lane_y = OP_BYTES + tr_base + ((tr_chunk ^ (brow0 >> 3)) << 4);
+  auto stage_base = [&](int lane, int s) {
+    int v = lane;
+    asm volatile("" : "+v"(v));  // (kept from being expanded outside the stage)
+    return v + (s & 1) * STAGE_BYTES;
+  };
+  auto tr8 = [&](int base, int m, int t) {
+    const char* p = smem + (base ^ (m << 5)) + 8 * t * ROW_BYTES;
+    short4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)p);
+    short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(p + 4 * ROW_BYTES));
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  auto read_frag = [&](Frag& f, int s, int kk) {
-    const char* st = smem + (s & 1) * STAGE_BYTES;
+  auto read_x = [&](bf16x8_t (&f)[NPB], int s, int t) {
+    const int base = stage_base(lane_x, s);
 #pragma unroll
-    for (int pb = 0; pb < NPB; ++pb) f.a[pb] = tr8(st, arow[pb], kk);
+    for (int pb = 0; pb < NPB; ++pb) f[pb] = tr8(base, pb, t);
+  };
+  auto read_y = [&](bf16x8_t (&f)[2], int base, int j) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) f.b[j] = tr8(st + OP_BYTES, brow[j], kk);
+    for (int t = 0; t < 2; ++t) f[t] = tr8(base, j, t);
   };
   // Rows >= nvalid of a stage contribute nothing: zero them in both the x
   // and the dy fragments (the clamped rows loaded there belong to the same
   // or, for an expert without rows, the previous expert; zeroing only one
   // operand would turn an Inf or NaN there into NaN instead of the exact
-  // zeros the gradient of an empty expert is).  Lane l holds rows
-  // 16 kk + 8 (l >> 5) + {0..3} and + 4 + {0..3}.
-  auto mask_frag = [&](Frag& f, int kk, int nvalid) {
-    // element i of the lane's 8 is row 16 kk + 8 (l >> 5) + i: kept if i < rem
-    const int rem = nvalid - 16 * kk - 8 * ((l >> 5) & 1);
-    uint32_t keep[4];
+  // zeros the gradient of an empty expert is).  Element i of the lane's 8 is
+  // row 16 g4 + 8 t + i.
+  auto mask = [&](bf16x8_t& f, int t, int nvalid) {
+    const int rem = nvalid - 16 * g4 - 8 * t;
+    u32x4_t v = __builtin_bit_cast(u32x4_t, f);
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
-      keep[d] = (2 * d < rem ? 0x0000ffffu : 0u) | (2 * d + 1 < rem ? 0xffff0000u : 0u);
-#pragma unroll
-    for (int pb = 0; pb < NPB; ++pb) {
-      u32x4_t v = __builtin_bit_cast(u32x4_t, f.a[pb]);
-#pragma unroll
-      for (int d = 0; d < 4; ++d) v[d] &= keep[d];
-      f.a[pb] = __builtin_bit_cast(bf16x8_t, v);
-    }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      u32x4_t v = __builtin_bit_cast(u32x4_t, f.b[j]);
-#pragma unroll
-      for (int d = 0; d < 4; ++d) v[d] &= keep[d];
-      f.b[j] = __builtin_bit_cast(bf16x8_t, v);
-    }
+    for (int d = 0; d < 4; ++d) v[d] &= (2 * d < rem ? 0x0000ffffu : 0u) | (2 * d + 1 < rem ? 0xffff0000u : 0u);
+    f = __builtin_bit_cast(bf16x8_t, v);
   };
 
   // ---- prologue --------------------------------------------------------------
-  issue(0);
-  issue(1);
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+    issue_prep(st);
+#pragma unroll
+    for (int i = 0; i < DMA_OP; ++i) issue_x(i);
+#pragma unroll
+    for (int i = 0; i < DMA_OP; ++i) issue_y(i);
+    issue_advance();
+  }
   wait_vm_barrier<DMA_PER_STAGE>();
-  Frag f0, f1;
-  read_frag(f0, 0, 0);
+  bf16x8_t fx[2][NPB], fy[4][2];  // dy block j in buffer j % 4
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    read_x(fx[t], 0, t);
+    read_y(fy[t], stage_base(lane_y, 0), t);
+  }
 
   int s = 0;
   for (int r = 0; r < nmy; ++r) {
     const Tile t = tile_of(r);
-    floatx16_t acc[NPB][NJ];
+    floatx4_t acc[NPB][NJ];
 #pragma unroll
     for (int i = 0; i < NPB; ++i)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-    auto mfma = [&](const Frag& f) {
-#pragma unroll
-      for (int j = 0; j < NJ; ++j)
+      for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    // One stage, dy block by dy block (8 MFMAs each), the dy fragments read
+    // two blocks ahead.
+    //   A (before block 2): every wave has read the stage's x rows; the
+    //     next-but-one stage's go out, one instruction per block.
+    //   B (before the last two blocks): every wave has read the whole stage
+    //     and the next one has landed (all but the DMA_OP instructions
+    //     issued at A); the next-but-one stage's dy rows follow.
+    // The first and last two blocks run k32 step by k32 step, while the next
+    // stage's first fragments are read.
+    auto stage = [&](auto maskedc, int nvalid) {
+      constexpr bool MASKED = decltype(maskedc)::value;
+      auto mfma_t = [&](int j, int tt) {
+        if constexpr (MASKED) mask(fy[j % 4][tt], tt, nvalid);
 #pragma unroll
         for (int pb = 0; pb < NPB; ++pb)
-          acc[pb][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[pb], f.b[j], acc[pb][j], 0, 0, 0);
+          acc[pb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fx[tt][pb], fy[j % 4][tt], acc[pb][j], 0, 0, 0);
+      };
+      const int yb = stage_base(lane_y, s);
+      static_for<0, 2>([&](auto tc) {
+        constexpr int tt = decltype(tc)::value;
+        if constexpr (MASKED) {
+#pragma unroll
+          for (int pb = 0; pb < NPB; ++pb) mask(fx[tt][pb], tt, nvalid);
+        }
+        read_y(fy[tt + 2], yb, tt + 2);
+        mfma_t(0, tt);
+        mfma_t(1, tt);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      lds_barrier();
+      issue_prep(s + 2);
+      static_for<2, NJ - 2>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        read_y(fy[(j + 2) % 4], yb, j + 2);
+        issue_x(j - 2);
+        mfma_t(j, 0);
+        mfma_t(j, 1);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      static_assert(NJ - 4 == DMA_OP, "one x instruction per block between the barriers");
+      wait_vm_barrier<DMA_OP>();
+      const int ybn = stage_base(lane_y, s + 1);
+      static_for<0, 2>([&](auto tc) {
+        constexpr int tt = decltype(tc)::value;
+        read_y(fy[tt], ybn, tt);
+        issue_y(2 * tt);
+        mfma_t(NJ - 2, tt);
+        issue_y(2 * tt + 1);
+        mfma_t(NJ - 1, tt);
+        __builtin_amdgcn_sched_barrier(0);
+        read_x(fx[tt], s + 1, tt);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      issue_advance();
+      ++s;
     };
-    for (int ks = 0; ks < t.nks; ++ks, ++s) {
-      const int nvalid = t.m1 - (t.m0 + TK * ks);
-      const bool partial = nvalid < TK;  // wave-uniform
-      if (partial) mask_frag(f0, 0, nvalid);
-      read_frag(f1, s, 1);
-      if (partial) mask_frag(f1, 1, nvalid);
-      mfma(f0);
-      read_frag(f0, s, 2);
-      if (partial) mask_frag(f0, 2, nvalid);
-      mfma(f1);
-      read_frag(f1, s, 3);
-      if (partial) mask_frag(f1, 3, nvalid);
-      mfma(f0);
-      wait_vm_barrier<0>();  // stage s + 1 landed, every wave done with stage s
-      issue(s + 2);
-      read_frag(f0, s + 1, 0);
-      mfma(f1);
-    }
+    // only a tile's last stage can be partial
+    const int nvalid = t.m1 - t.m0 - TK * (t.nks - 1);
+    for (int ks = nvalid < TK ? 1 : 0; ks < t.nks; ++ks) stage(std::false_type{}, TK);
+    if (nvalid < TK) stage(std::true_type{}, nvalid);
 
     // ---- split leftover tile: publish this piece's sums; the last piece to
     //      arrive adds all of them in piece order and runs the epilogue.
@@ -278,7 +337,7 @@ __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDma
     //      the arrival is counted, and the last piece invalidates its caches
     //      (acquire) before it reads the others'; it resets the counter.
     if (np > 1 && r >= nfull) {
-      constexpr int NV4 = NPB * NJ * 4;                   // float4 per lane
+      constexpr int NV4 = NPB * NJ;                       // float4 per lane
       constexpr uint32_t WAVE_BYTES = NV4 * 64 * 16;      // 32 KB
       constexpr uint64_t PIECE_BYTES = (uint64_t)WAVES * WAVE_BYTES;  // 256 KB
       static_assert(PIECE_BYTES <= kSplitPartBytes, "partial of a piece");
@@ -294,10 +353,7 @@ __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDma
       for (int pb = 0; pb < NPB; ++pb)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            *(gfloatx4_t*)(mine + (uint32_t)(((pb * NJ + j) * 4 + g) * 1024) + loff) =
-                floatx4_t{acc[pb][j][4 * g], acc[pb][j][4 * g + 1], acc[pb][j][4 * g + 2], acc[pb][j][4 * g + 3]};
+          *(gfloatx4_t*)(mine + (uint32_t)((pb * NJ + j) * 1024) + loff) = acc[pb][j];
       wait_vm<0>();  // this wave's partial has reached L2; every DMA has landed
       __syncthreads();
       // (the stage buffers are idle: no DMA is issued after the last unit)
@@ -322,34 +378,26 @@ __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDma
 #pragma unroll
       for (int pb = 0; pb < NPB; ++pb)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) acc[pb][j][v] = 0.f;
-      // the sum in piece order, one 16-float block (four loads) at a time
+        for (int j = 0; j < NJ; ++j) acc[pb][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+      // the sum in piece order, four blocks (loads) at a time
       for (int jp = 0; jp < np; ++jp) {
         const uint64_t src = piece(jp);
 #pragma unroll
-        for (int pb = 0; pb < NPB; ++pb)
+        for (int j = 0; j < NJ; ++j) {
+          floatx4_t v[NPB];
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) {
-            floatx4_t v[4];
+          for (int pb = 0; pb < NPB; ++pb) v[pb] = *(const gfloatx4_t*)(src + (uint32_t)((pb * NJ + j) * 1024) + loff);
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
-              v[g] = *(const gfloatx4_t*)(src + (uint32_t)(((pb * NJ + j) * 4 + g) * 1024) + loff);
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-              for (int i = 0; i < 4; ++i) acc[pb][j][4 * g + i] += v[g][i];
-            __builtin_amdgcn_sched_barrier(0);
-          }
+          for (int pb = 0; pb < NPB; ++pb) acc[pb][j] += v[pb];
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
 
-    // ---- epilogue: acc[pb][j][4g + i] = dw[e][n][k], n = nt*TQ + brow[j] +
-    //      lane % 32, k = kt*TP + arow[pb] + 8g + 4 (lane / 32) + i.
-    int er32 = l & 31;
-    asm volatile("" : "+v"(er32));
-    const int half = l >> 5;
+    // ---- epilogue: acc[pb][j][i] = dw[e][n][k], n = nt*TQ + brow0 + 16 j +
+    //      lane % 16, k = kt*TP + arow0 + 16 pb + 4 (lane / 16) + i.
+    int er16 = r16;
+    asm volatile("" : "+v"(er16));
     // Both forms go through the wave's private 4 KB LDS slab (row r: 128
     // bytes, 16-byte chunk c at c ^ (r & 7)) and leave as streaming stores
     // of 8 whole 128-byte rows per instruction: the gradient is written once
@@ -360,16 +408,17 @@ __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDma
     if (a.dw_fp32) {
       // fp32: one 32-row x 32-column block (128 bytes per row) at a time
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
+      for (int j = 0; j < NJ; j += 2) {
 #pragma unroll
-        for (int pb = 0; pb < NPB; ++pb) {
-          if (t.kt * TP + arow[pb] < a.K) {  // wave-uniform: the block's 32 columns are valid together
-            const floatx16_t& v = acc[pb][j];
+        for (int pb = 0; pb < NPB; pb += 2) {
+          if (t.kt * TP + arow0 + 16 * pb < a.K) {  // wave-uniform: the block's 32 columns are valid together
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const int chunk = (2 * g + half) ^ (er32 & 7);  // columns 8g + 4 half .. + 3
-              *(float4*)(slab + er32 * 128 + chunk * 16) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
-            }
+            for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+              for (int p = 0; p < 2; ++p) {
+                const int row = 16 * jj + er16, chunk = (4 * p + g4) ^ (er16 & 7);  // columns 16 p + 4 g4 .. + 3
+                *(floatx4_t*)(slab + row * 128 + chunk * 16) = acc[pb + p][j + jj];
+              }
             lds_wait();  // the slab writes have landed
             uint4 o4[4];
 #pragma unroll
@@ -378,30 +427,30 @@ __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDma
               o4[i] = *(const uint4*)(slab + r * 128 + (((l & 7) ^ (r & 7)) << 4));
             }
             lds_wait();  // read before the next block overwrites the slab
-            const int col = t.kt * TP + arow[pb] + 4 * (l & 7);
+            const int col = t.kt * TP + arow0 + 16 * pb + 4 * (l & 7);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const int n = t.nt * TQ + brow[j] + 8 * i + (l >> 3);
+              const int n = t.nt * TQ + brow0 + 16 * j + 8 * i + (l >> 3);
               if (n < a.N) store_stream((uint4*)((float*)a.dw + ((int64_t)t.e * a.N + n) * a.K + col), o4[i]);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
-    } else if (t.kt * TP + arow[0] < a.K) {  // the wave's 64 columns are valid together
+    } else if (t.kt * TP + arow0 < a.K) {  // the wave's 64 columns are valid together
       // bf16: one 32-row block (the wave's 64 columns, 128 bytes per row)
       // at a time
-      const int col = t.kt * TP + arow[0] + 8 * (l & 7);
+      const int col = t.kt * TP + arow0 + 8 * (l & 7);
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
+      for (int j = 0; j < NJ; j += 2) {
 #pragma unroll
-        for (int pb = 0; pb < NPB; ++pb)
+        for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const floatx16_t& v = acc[pb][j];
-            const int chunk = (4 * pb + g) ^ (er32 & 7);
-            *(uint2*)(slab + er32 * 128 + chunk * 16 + half * 8) =
-                make_uint2(pack_bf16x2(v[4 * g], v[4 * g + 1]), pack_bf16x2(v[4 * g + 2], v[4 * g + 3]));
+          for (int pb = 0; pb < NPB; ++pb) {
+            const floatx4_t& v = acc[pb][j + jj];
+            const int row = 16 * jj + er16, chunk = (2 * pb + (g4 >> 1)) ^ (er16 & 7);
+            *(uint2*)(slab + row * 128 + chunk * 16 + (g4 & 1) * 8) =
+                make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
           }
         lds_wait();  // the slab writes have landed
         uint4 o4[4];
@@ -413,10 +462,8 @@ __global__ __launch_bounds__(THREADS, 1) void gg_wgrad_dma_kernel(const WgradDma
         lds_wait();  // read before the next block overwrites the slab
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int r = 8 * i + (l >> 3);
-          const uint4 o = o4[i];
-          const int n = t.nt * TQ + brow[j] + r;
-          if (n < a.N) store_stream((uint4*)((bf16_t*)a.dw + ((int64_t)t.e * a.N + n) * a.K + col), o);
+          const int n = t.nt * TQ + brow0 + 16 * j + 8 * i + (l >> 3);
+          if (n < a.N) store_stream((uint4*)((bf16_t*)a.dw + ((int64_t)t.e * a.N + n) * a.K + col), o4[i]);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
