@@ -93,6 +93,70 @@ def test_small_shared_expert(ops, T, D, H):
     assert_close(to_np(out), base + y, TOL, "out")
 
 
+# rows per expert, N (or H), K (a multiple of 128) of the fp8 form
+FP8_CASES = [
+    ((1,), 128, 128),                                 # one row, one k stage
+    ((0, 1, 0, 2, 1), 192, 4096),                    # 64 x 128 tiles, up rows straddle scale blocks, rotated k walk
+    ((64, 65, 33, 1, 0, 17, 16, 63), 320, 384),      # 64-row tiles and one row past, 16-row block edges
+    ((9,) * 200 + (0,) * 20 + (64,) * 3, 1152, 256),   # 64 x 256 tiles, half-full last tile
+    ((128, 129, 97, 1, 300, 0, 31), 448, 640),       # 128 x 128 tiles, one row past
+    ((90, 100, 128, 70, 96) * 26, 1152, 512),          # 128 x 256 tiles, whole and partial rounds
+]
+
+
+@pytest.mark.parametrize("i", range(len(FP8_CASES)))
+def test_small_fp8(ops, i):
+    """Every epilogue of the fp8 small tiles against the dequantising oracle
+    (operands e4m3 with fp32 block scales, so only the sums' fp32 rounding
+    and the output's bf16 rounding differ)."""
+    counts, n, K = FP8_CASES[i]
+    counts = np.array(counts, np.int64)
+    M, E = int(counts.sum()), len(counts)
+    offs_h, od = np.cumsum(counts), _offs(counts)
+    rng = np.random.default_rng(200 + i)
+    H, N = -(-n // 64) * 64, -(-n // 128) * 128
+    x = bf16_dev(rand_bf16(rng, (M, K)))
+    announce(f"small fp8 M={M} E={E} n={n} K={K}")
+    xq, sx = ops.quantize_fp8_rows(x)
+    xd = O.e4m3_bits_to_f32(xq.cpu().numpy()).reshape(M, K // 128, 128) * sx.cpu().numpy().T[:, :, None]
+    xd = xd.reshape(M, K)
+
+    def weights(rows):
+        w = bf16_dev(rand_bf16(rng, (E, rows, K), 0.05))
+        q, s = ops.quantize_fp8_blocks(w)
+        d = O.e4m3_bits_to_f32(q.cpu().numpy()).reshape(E, rows // 128, 128, K // 128, 128)
+        return q, s, (d * s.cpu().numpy()[:, :, None, :, None]).reshape(E, rows, K)
+
+    wq, sw, wd = weights(N)
+    y = O.grouped_mm(xd, wd, offs_h)
+    assert_close(to_np(ops.grouped_mm_fp8(xq, sx, wq, sw, od)), y, TOL, "store")
+    dest, scale = rng.permutation(M).astype(np.int32), rng.random(M).astype(np.float32)
+    out = ops.grouped_mm_fp8_unpermute(xq, sx, wq, sw, od, f32_dev(scale), torch.from_numpy(dest).to(DEV), M)
+    ref = np.zeros((M, N), np.float32)
+    ref[dest] = y * scale[:, None]
+    assert_close(to_np(out), ref, TOL, "scatter")
+    wq, sw, wd = weights(2 * H)
+    h_ref = O.bf16_round(O.grouped_mm(xd, wd, offs_h))
+    for limit in (None, 0.5):
+        a, h = ops.grouped_mm_fp8_swiglu(xq, sx, wq, sw, od, limit, save_h=True)
+        assert_close(to_np(h), h_ref, TOL, "h")
+        assert_close(to_np(a), O.swiglu(h_ref, limit), 2 * TOL, "a")
+
+
+@pytest.mark.parametrize("R", [1, 4, 5, 8191, 8193])
+def test_fp8_row_quantiser_row_groups(ops, R):
+    """Few rows run one per wave, many four per wave: the same codes and
+    scales either way (the rows of a larger call)."""
+    rng = np.random.default_rng(R)
+    K = 256
+    x = bf16_dev(rand_bf16(rng, (R, K)))
+    big = torch.cat([x, bf16_dev(rand_bf16(rng, (20000, K)))])
+    announce(f"fp8 row quantiser R={R}")
+    q, s = ops.quantize_fp8_rows(x)
+    q2, s2 = ops.quantize_fp8_rows(big)
+    assert torch.equal(q, q2[:R]) and torch.equal(s, s2[:, :R])
+
+
 def test_large_tiles_split_epilogues_and_replay(ops):
     """35 experts of 320 rows keep the 320 x 256 kernel, whose 24 leftover
     tiles (of 280) are cut along k: the SwiGLU epilogue (with and without the

@@ -86,7 +86,8 @@ void probe_chain_arm(const hipEvent_t* events, int n_launches) {
 }
 
 // Weight rows per tile if a forward GEMM over `cols` weight rows per expert
-// takes the small-tile kernel, 0 if the 320 x 256 kernel.
+// takes the small-tile kernel, 0 if the large one (large_rows x 256: 320 rows
+// in bf16, 256 in fp8).
 //
 // Up to kSmallAvgRows rows per expert on average the GEMM streams weights
 // and the small tiles' deeper ring is ahead (Qwen3-30B-A3B experts, both
@@ -101,7 +102,7 @@ void probe_chain_arm(const hipEvent_t* events, int n_launches) {
 // rows 98 -> 57 us and 8000 rows 121 us against 133 (kept large), while two
 // or more rounds of large tiles are better left alone (Llama4-Scout, 128
 // rows per expert: 568 us against 664).
-static int small_tile_cols(int M, int E, int64_t cols) {
+static int small_tile_cols(int M, int E, int64_t cols, int large_rows) {
   const int rows = small_tile_rows(M, E);
   if (rows == 0) return 0;
   const int64_t G = (num_cus() + 7) & ~7;
@@ -116,7 +117,7 @@ static int small_tile_cols(int M, int E, int64_t cols) {
   const int64_t c128 = cost(rows, 128, rows == 64 ? 50 : 66), c256 = cost(rows, 256, rows == 64 ? 85 : 108);
   const int small = c128 < c256 ? 128 : 256;
   if (M <= kSmallAvgRows * (int64_t)E) return small;
-  return tiles(kFwdTileRows, 256) < 2 * G && std::min(c128, c256) < cost(kFwdTileRows, 256, 200) ? small : 0;
+  return tiles(large_rows, 256) < 2 * G && std::min(c128, c256) < cost(large_rows, 256, 200) ? small : 0;
 }
 
 // plan: the tile plan; part: the partial-sum area of split leftover tiles
@@ -129,7 +130,7 @@ static hipError_t fwd(int epi, FwdGemm g, const int* offs, int E, int M, void* p
     if (err != hipSuccess) return err;
   }
   const TileTable tt = tile_table_in(plan, M, E);
-  const int small = small_tile_cols(M, E, epi == EPI_SWIGLU ? 2 * (int64_t)g.n : g.n);
+  const int small = small_tile_cols(M, E, epi == EPI_SWIGLU ? 2 * (int64_t)g.n : g.n, kFwdTileRows);
   g.table = small ? tt.small_table : tt.table;
   g.n_qtiles = small ? tt.small_count : tt.count;
   g.split_cnt = tt.split_cnt;
@@ -239,12 +240,13 @@ hipError_t launch_moe_experts_forward(const void* tokens, int T, int D, int H, i
 // ---- fp8 forward (gemm_fp8.hip) ----------------------------------------------
 static hipError_t fp8(int epi, Fp8Args a, const int* offs, int E, int M, void* ws,
                       hipStream_t stream) {
-  hipError_t err = launch_tile_map(offs, E, M, kFp8TileRows, ws, false, stream);
+  hipError_t err = launch_tile_map(offs, E, M, kFp8TileRows, ws, true, stream);
   if (err != hipSuccess) return err;
   const TileTable tt = tile_table_in(ws, M, E);
-  a.table = tt.table;
-  a.n_qtiles = tt.count;
-  return launch_fp8_gemm(epi, a, stream);
+  const int small = small_tile_cols(M, E, a.n_p, kFp8TileRows);
+  a.table = small ? tt.small_table : tt.table;
+  a.n_qtiles = small ? tt.small_count : tt.count;
+  return small ? launch_small_fp8_gemm(epi, a, tt.small_rows, small, stream) : launch_fp8_gemm(epi, a, stream);
 }
 
 static Fp8Args fp8_args(const void* xq, const float* sx, const void* wq, const float* sw, int M,

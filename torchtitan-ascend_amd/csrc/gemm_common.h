@@ -313,5 +313,7 @@ hipError_t launch_small_gemm(int epi, FwdArgs a, int tile_rows, int tile_cols, h
 hipError_t launch_dgrad_gemm(int epi, const DgradGemm& g, hipStream_t stream);
 // fp8 forward GEMM over a tile table of at most kFp8TileRows rows per tile.
 hipError_t launch_fp8_gemm(int epi, const Fp8Args& a, hipStream_t stream);
+// Small-tile form (gemm_fp8_small.hip): tiles of at most `rows` token rows, `cols` weight rows.
+hipError_t launch_small_fp8_gemm(int epi, const Fp8Args& a, int rows, int cols, hipStream_t stream);
 
 }  // namespace ttamd

@@ -13,6 +13,7 @@
 // hardware conversion instructions' saturation mode.  |v| above 464 (half
 // way to 480) gives NaN, which the absmax / 448 recipe never produces.
 #include "common.h"
+#include "gemm_common.h"
 #include "kernels.h"
 
 namespace ttamd {
@@ -44,7 +45,8 @@ __device__ __forceinline__ bool e4m3_tie_risk(float q) {
 }
 
 // ---------------------------------------------------------------------------
-// Rows: a workgroup of 4 waves quantises 16 rows (4 per wave).  Lane l holds
+// Rows: a workgroup of 4 waves quantises 16 rows (4 per wave), or 4 where
+// there are few.  Lane l holds
 // 8 consecutive channels of every 512-channel step (16 lanes form one
 // 128-channel block).  All of a row's loads are issued before any of its
 // arithmetic (up to kMaxSteps x 16 bytes per lane), so a wave keeps its whole
@@ -56,23 +58,24 @@ __device__ __forceinline__ bool e4m3_tie_risk(float q) {
 // even, OCP e4m3) packs the bytes: the result is the IEEE quotient's cast,
 // bit for bit, at a fraction of the VALU work of a division per element.
 // ---------------------------------------------------------------------------
-constexpr int kQRows = 16;
+constexpr int kQRows = 16;     // rows per workgroup at most
+constexpr int kQRowsFew = 4;   // ... where 16 would leave most CUs idle
 constexpr int kMaxKBlocks = 64;  // K <= 8192
 constexpr int kMaxSteps = kMaxKBlocks / 4;  // 512-channel steps per row
 
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const uint4* __restrict__ in,
                                                             const int* __restrict__ src_index,
                                                             int src_div, const float* __restrict__ row_mul,
-                                                            int n_in, int R, int K,
+                                                            int n_in, int R, int K, int rows_wg,
                                                             uint2* __restrict__ q_out,
                                                             float* __restrict__ scale_t) {
   __shared__ float sc[kMaxKBlocks][kQRows];
   const int w = threadIdx.x >> 6;
   const int l = threadIdx.x & 63;
-  const int row_base = blockIdx.x * kQRows;
+  const int row_base = blockIdx.x * rows_wg;
   const int kv = K / 8;  // 16-byte vectors per row
   const int nkb = K / 128;
-  for (int rr = w; rr < kQRows; rr += 4) {
+  for (int rr = w; rr < rows_wg; rr += 4) {
     const int row = row_base + rr;
     if (row >= R) break;
     int src = row;
@@ -128,9 +131,11 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const uint4* __restr
     }
   }
   __syncthreads();
-  // scale_t[kb][row_base .. row_base + 15]
-  for (int i = threadIdx.x; i < nkb * kQRows; i += 256) {
-    const int kb = i / kQRows, rr = i % kQRows;
+  // scale_t[kb][row_base .. row_base + rows_wg - 1]
+  const int sh = rows_wg == kQRows ? 4 : 2;
+  static_assert(kQRows == 1 << 4 && kQRowsFew == 1 << 2, "shift");
+  for (int i = threadIdx.x; i < nkb << sh; i += 256) {
+    const int kb = i >> sh, rr = i & (rows_wg - 1);
     if (row_base + rr < R) scale_t[(int64_t)kb * R + row_base + rr] = sc[kb][rr];
   }
 }
@@ -177,9 +182,12 @@ __global__ __launch_bounds__(256) void quantize_blocks_kernel(const uint4* __res
 hipError_t launch_quantize_rows(const void* in, const int* src_index, int src_div, const float* row_mul,
                                 int n_in, int R, int K, void* q_out, float* scale_t, hipStream_t stream) {
   if (R == 0) return hipSuccess;
-  const int grid = (R + kQRows - 1) / kQRows;
+  // 16 rows per workgroup make one 64-byte scale store per k-block; below two
+  // workgroups per CU one row per wave is ahead (200 rows of 7168, gathered: 18 -> 13 us)
+  const int rows_wg = R > 2 * kQRows * num_cus() ? kQRows : kQRowsFew;
+  const int grid = (R + rows_wg - 1) / rows_wg;
   return launch_k(false, quantize_rows_kernel, dim3(grid), dim3(256), 0, stream, (const uint4*)in, src_index,
-                  src_div, row_mul, n_in, R, K, (uint2*)q_out, scale_t);
+                  src_div, row_mul, n_in, R, K, rows_wg, (uint2*)q_out, scale_t);
 }
 
 hipError_t launch_quantize_blocks(const void* w, int E, int N, int K, void* q_out, float* scale,
