@@ -42,7 +42,8 @@ constexpr int RWAVES = 4;   // one 32-token block per wave
 constexpr int RTHREADS = 64 * RWAVES;
 constexpr int RTK = 64;     // k per stage: 128-byte rows
 constexpr int kRouterMaxE = 256;
-constexpr int kRouterMaxSplits = 4;  // slices of D (partial logits per token and expert)
+constexpr int kRouterMaxSplits = 4;   // slices of D (partial logits per token and expert)
+constexpr int kRouterFewSplits = 16;  // ... of calls with few tokens
 
 // Stage buffers of the gate GEMM: as many as fit (at most 6).
 template <int EB>
@@ -221,45 +222,47 @@ __global__ __launch_bounds__(256) void router_topk_partials_kernel(const RouterT
   const int E = FULL ? 16 * PL : a.E;
   auto eid = [&](int m) { return G * gi + m % G + 16 * G * (m / G); };
   auto live = [&](int m) { return FULL || eid(m) < E; };
-  // every partial first (one batch of independent loads), then the sums in
-  // split order
-  float pv[kRouterMaxSplits][PL];
+  // the partials of kRouterMaxSplits slices at a time (one batch of
+  // independent loads), summed in split order
   const bool vec = FULL || (E % G) == 0;  // runs never straddle E and stay aligned
-#pragma unroll
-  for (int s = 0; s < kRouterMaxSplits; ++s)
-#pragma unroll
-    for (int m0 = 0; m0 < PL; m0 += G) {
-      const int e0 = eid(m0);
-      const float* src = a.part + ((int64_t)s * a.T + tt) * E + e0;
-      if (s < a.S && vec && (FULL || e0 < E)) {
-        if constexpr (G == 4) {
-          const float4 v = *(const float4*)src;
-          pv[s][m0] = v.x; pv[s][m0 + 1] = v.y; pv[s][m0 + 2] = v.z; pv[s][m0 + 3] = v.w;
-        } else if constexpr (G == 2) {
-          const float2 v = *(const float2*)src;
-          pv[s][m0] = v.x; pv[s][m0 + 1] = v.y;
-        } else {
-          pv[s][m0] = src[0];
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < G; ++i) pv[s][m0 + i] = (s < a.S && e0 + i < E) ? src[i] : 0.f;
-      }
-    }
   float sc[PL];
+  for (int s0 = 0; s0 < a.S; s0 += kRouterMaxSplits) {  // one pass but for few tokens
+    float pv[kRouterMaxSplits][PL];
+#pragma unroll
+    for (int s = 0; s < kRouterMaxSplits; ++s)
+#pragma unroll
+      for (int m0 = 0; m0 < PL; m0 += G) {
+        const int e0 = eid(m0);
+        const float* src = a.part + ((int64_t)(s0 + s) * a.T + tt) * E + e0;
+        if (s0 + s < a.S && vec && (FULL || e0 < E)) {
+          if constexpr (G == 4) {
+            const float4 v = *(const float4*)src;
+            pv[s][m0] = v.x; pv[s][m0 + 1] = v.y; pv[s][m0 + 2] = v.z; pv[s][m0 + 3] = v.w;
+          } else if constexpr (G == 2) {
+            const float2 v = *(const float2*)src;
+            pv[s][m0] = v.x; pv[s][m0 + 1] = v.y;
+          } else {
+            pv[s][m0] = src[0];
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < G; ++i) pv[s][m0 + i] = (s0 + s < a.S && e0 + i < E) ? src[i] : 0.f;
+        }
+      }
+#pragma unroll
+    for (int m = 0; m < PL; ++m) {
+      float z = s0 == 0 ? pv[0][m] : sc[m] + pv[0][m];
+#pragma unroll
+      for (int s = 1; s < kRouterMaxSplits; ++s)
+        if (s0 + s < a.S) z += pv[s][m];
+      sc[m] = z;
+    }
+  }
   float mx = -INFINITY;
 #pragma unroll
   for (int m = 0; m < PL; ++m) {
-    float z = -INFINITY;
-    if (live(m)) {
-      z = pv[0][m];
-#pragma unroll
-      for (int s = 1; s < kRouterMaxSplits; ++s)
-        if (s < a.S) z += pv[s][m];
-      z = round_bf16(z);
-    }
-    sc[m] = z;
-    mx = fmaxf(mx, z);
+    sc[m] = live(m) ? round_bf16(sc[m]) : -INFINITY;
+    mx = fmaxf(mx, sc[m]);
   }
   if (a.logits && valid) {
     bf16_t* lrow = a.logits + (int64_t)t * E;
@@ -522,12 +525,16 @@ hipError_t launch_gemm_eb(const RouterGemmArgs& a, int S, hipStream_t stream) {
 // Slices of D: enough gate-GEMM workgroups to give every CU one (each CU
 // then moves T*D*2/CUs bytes of x plus E*D*2/S of the weight), at most
 // kRouterMaxSplits (the partial logits cost 8*S*T*E bytes of traffic), each
-// slice at least 4 stages (256 columns) long.
+// slice at least 4 stages (256 columns) long.  Up to 2 token tiles the
+// partials are small and a slice's length is what a call waits for: up to
+// kRouterFewSplits slices of at least 2 stages (32 tokens, D = 2048, E = 128:
+// 8.5 -> 5.2 us).
 int router_splits(int T, int D) {
   const int tiles = (T + RT - 1) / RT;
   const int stages = D / RTK;
   int S = (num_cus() + tiles - 1) / tiles;
-  S = max(1, min(min(S, kRouterMaxSplits), stages / 4));
+  S = tiles <= 2 ? min(min(S, kRouterFewSplits), stages / 2) : min(min(S, kRouterMaxSplits), stages / 4);
+  S = max(1, S);
   const int per = (stages + S - 1) / S;
   return (stages + per - 1) / per;  // no empty slice
 }
