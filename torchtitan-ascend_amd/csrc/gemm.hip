@@ -95,14 +95,16 @@ void probe_chain_arm(const hipEvent_t* events, int n_launches) {
 // rows 299 -> 251, 96 rows 315 -> 281; DeepSeek-V3's 94 rows 632 -> 530); at
 // 125-128 rows many experts need a second 128-row tile and it is not (331 ->
 // 337 us, 664 -> 680 us).  With more rows per expert it pays where the large
-// tiles leave the chip idle in their last round: the rounds of each tiling
-// are weighed with its time per 64-k stage (measured on whole rounds:
-// 2.0 us for 320 x 256, 1.08 for 128 x 256, 0.66 for 128 x 128, 0.85 for
-// 64 x 256 and 0.5 for 64 x 128), e.g. 4 experts of 2048 x 1024 with 2000
-// rows 98 -> 57 us and 8000 rows 121 us against 133 (kept large), while two
-// or more rounds of large tiles are better left alone (Llama4-Scout, 128
-// rows per expert: 568 us against 664).
-static int small_tile_cols(int M, int E, int64_t cols, int large_rows) {
+// tiles leave the chip idle in their last round and the weights are re-read
+// from the memory-side cache (256 MB): the rounds of each tiling are weighed
+// with its time per 64-k stage (measured on whole rounds: 2.0 us for 320 x
+// 256, 1.08 for 128 x 256, 0.66 for 128 x 128, 0.85 for 64 x 256 and 0.5 for
+// 64 x 128), e.g. 4 experts of 2048 x 1024 with 2000 rows 98 -> 57 us, with
+// 8000 rows 121 us against 133 (kept large).  Weights that stream from HBM
+// or two and more rounds of large tiles are better left alone (Llama4-Scout
+// w2, 128 rows per expert: 348 us against 388; w13 568 against 664).
+constexpr int64_t kSmallWeightBytes = 256 << 20;
+static int small_tile_cols(int M, int E, int64_t cols, int64_t row_bytes, int large_rows) {
   const int rows = small_tile_rows(M, E);
   if (rows == 0) return 0;
   const int64_t G = (num_cus() + 7) & ~7;
@@ -117,7 +119,10 @@ static int small_tile_cols(int M, int E, int64_t cols, int large_rows) {
   const int64_t c128 = cost(rows, 128, rows == 64 ? 50 : 66), c256 = cost(rows, 256, rows == 64 ? 85 : 108);
   const int small = c128 < c256 ? 128 : 256;
   if (M <= kSmallAvgRows * (int64_t)E) return small;
-  return tiles(large_rows, 256) < 2 * G && std::min(c128, c256) < cost(large_rows, 256, 200) ? small : 0;
+  return std::min(E, M) * cols * row_bytes <= kSmallWeightBytes && tiles(large_rows, 256) < 2 * G &&
+                 std::min(c128, c256) < cost(large_rows, 256, 200)
+             ? small
+             : 0;
 }
 
 // plan: the tile plan; part: the partial-sum area of split leftover tiles
@@ -130,7 +135,7 @@ static hipError_t fwd(int epi, FwdGemm g, const int* offs, int E, int M, void* p
     if (err != hipSuccess) return err;
   }
   const TileTable tt = tile_table_in(plan, M, E);
-  const int small = small_tile_cols(M, E, epi == EPI_SWIGLU ? 2 * (int64_t)g.n : g.n, kFwdTileRows);
+  const int small = small_tile_cols(M, E, epi == EPI_SWIGLU ? 2 * (int64_t)g.n : g.n, 2 * (int64_t)g.kred, kFwdTileRows);
   g.table = small ? tt.small_table : tt.table;
   g.n_qtiles = small ? tt.small_count : tt.count;
   g.split_cnt = tt.split_cnt;
@@ -243,7 +248,7 @@ static hipError_t fp8(int epi, Fp8Args a, const int* offs, int E, int M, void* w
   hipError_t err = launch_tile_map(offs, E, M, kFp8TileRows, ws, true, stream);
   if (err != hipSuccess) return err;
   const TileTable tt = tile_table_in(ws, M, E);
-  const int small = small_tile_cols(M, E, a.n_p, kFp8TileRows);
+  const int small = small_tile_cols(M, E, a.n_p, a.kred, kFp8TileRows);
   a.table = small ? tt.small_table : tt.table;
   a.n_qtiles = small ? tt.small_count : tt.count;
   return small ? launch_small_fp8_gemm(epi, a, tt.small_rows, small, stream) : launch_fp8_gemm(epi, a, stream);
