@@ -218,6 +218,7 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     }
   };
   int d_r = -1;  // tile round whose addresses are loaded
+  int d_rot = 0;  // its first k stage
   int d_qblk8 = 0;  // 8-row token blocks the MFMA reads: 4 * ceil(rows / 32)
   int d_pmax = 0, d_qmax = 0;  // last valid weight / token row of the tile (tile-relative)
   uint64_t d_pbase = 0, d_qbase = 0;
@@ -282,6 +283,14 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
         if (a.row_scale) dma4(q * 4, (uint64_t)(a.row_scale + ti.y), m + TQ * 4);
       }
     }
+    // Weight rows a multiple of 4 KB apart: tiles at the same k ask the same
+    // HBM channels, so each expert starts its k walk elsewhere (the tiles of
+    // one expert keep sharing their lines).  128 rows per expert of 768 x
+    // 2048, where the weights' stream is the bound: w13 197 -> 161 us; 256
+    // rows 233 -> 223, 512 rows unchanged; offsets per weight tile as well
+    // lose the shared token lines (512 rows 382 -> 407).  A split tile's
+    // pieces keep their k ranges.
+    if constexpr (!PT) d_rot = (a.ldp * 2) % 4096 == 0 && r < nfull ? U(3 * ti.x % ksteps) : 0;
     d_r = r;
   };
   // A stage's DMA is issued in two parts: the weight rows (P) at the stage
@@ -294,8 +303,9 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
   // Past the end the last stage is issued again.
   int n_r = 0, n_ks = nfull > 0 ? 0 : pc_k0, n_kend = nfull > 0 ? ksteps : pc_k1, n_left = total;
   auto issue_prep = [&](int s) {
-    const int r = n_r, ks = n_ks;
-    if (r != d_r) dma_tile(r);
+    if (n_r != d_r) dma_tile(n_r);
+    int ks = n_ks + d_rot;
+    ks = ks >= ksteps ? ks - ksteps : ks;
     d_spb = d_pbase + (PT ? (uint64_t)ks * TK * a.ldp * 2 : (uint64_t)ks * ROW_BYTES);
     d_sqb = d_qbase + (uint64_t)ks * ROW_BYTES;
     d_sst = lds0 + (uint32_t)((s & 1) * STAGE_BYTES) + w * 1024;
