@@ -188,4 +188,6 @@ def check(rc: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args))
+    rc = getattr(_lib if _lib is not None else load(), name)(*args)
+    if rc != 0:
+        check(rc)

@@ -47,6 +47,11 @@ hipError_t launch_k(bool gemm, F kernel, dim3 grid, dim3 block, uint32_t shmem, 
     e1 = p.gemm_end;
     p.gemm_start = p.gemm_end = nullptr;
   }
+  if (e0 == nullptr && e1 == nullptr) {
+    // (the plain launch costs the host ~0.9 us less)
+    kernel<<<grid, block, shmem, stream>>>(args...);
+    return hipGetLastError();
+  }
   hipExtLaunchKernelGGL(kernel, grid, block, shmem, stream, e0, e1, 0, args...);
   return hipGetLastError();
 }

@@ -24,12 +24,19 @@ from . import _lib
 _BF16 = torch.bfloat16
 
 
-def _p(t: torch.Tensor | None) -> ctypes.c_void_p | None:
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+def _p(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
-def _stream(dev: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+# torch's current stream of a device as a plain handle (0.1 us; building the
+# Stream object takes 1.8 us of a call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(dev: torch.device | str) -> int:
+    if _raw_stream is None or not isinstance(dev, torch.device) or dev.index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(dev.index)
 
 
 def _gpu(name: str, t: torch.Tensor) -> torch.device:
@@ -145,7 +152,7 @@ def router_fused(
     return_logits, the bf16 logits [T, E] as a third element.
     """
     dev = _gpu("x", x)
-    x = _want("x", x.reshape(-1, x.shape[-1]), _BF16)
+    x = _want("x", x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), _BF16)
     w_router = _want("w_router", w_router, _BF16)
     T, D = x.shape
     E, D2 = w_router.shape
@@ -240,7 +247,7 @@ def router_route(
             "router_route is the inference path (its scores carry no autograd); for training use "
             "functional.router (differentiable) followed by route"
         )
-    x = _want("x", x.reshape(-1, x.shape[-1]), _BF16)
+    x = _want("x", x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), _BF16)
     w_router = _want("w_router", w_router, _BF16)
     T, D = x.shape
     E, D2 = w_router.shape
@@ -307,11 +314,12 @@ def experts_forward(
     if r.sorted_indices.numel() != T * top_k:
         raise ValueError("routing does not match T * top_k rows")
     lib = _lib.load()
+    offsets = r.offsets.contiguous()  # inclusive offsets: its int32 entries from the second on
     out = torch.empty(T, D, dtype=_BF16, device=dev)
     ws = _ws(lib.ttamd_moe_experts_forward_workspace_bytes(T, D, H, E, top_k, int(bool(score_before_experts))), dev)
     plan = r.plan
     _lib.call(
-        "ttamd_moe_experts_forward", _p(x), T, D, H, E, top_k, _p(r.sorted_indices), _p(r.offs.contiguous()),
+        "ttamd_moe_experts_forward", _p(x), T, D, H, E, top_k, _p(r.sorted_indices), _p(offsets) + 4,
         _p(r.sorted_scores), int(bool(score_before_experts)), _limit(swiglu_limit), _p(w13), _p(w2), _p(out),
         _p(plan), 0 if plan is None else plan.numel(), _p(ws), ws.numel(), _stream(dev),
     )
