@@ -104,19 +104,39 @@ FP8_CASES = [
 ]
 
 
+# The same of the 256 x 256 fp8 tiles: every 16-row block count in both halves,
+# walks of 1 to 4 tiles per workgroup, with 1 to 3 k stages of 128
+FP8_HEIGHTS = (1, 16, 17, 40, 64, 97, 128, 129, 144, 161, 200, 230, 256, 257, 300, 512)
+FP8_LARGE_CASES = [
+    (FP8_HEIGHTS * 4, 3072, 128),
+    (FP8_HEIGHTS * 4, 1152, 256),
+    (FP8_HEIGHTS[::-1] * 4, 1024, 384),
+]
+
+
 @pytest.mark.parametrize("i", range(len(FP8_CASES)))
 def test_small_fp8(ops, i):
     """Every epilogue of the fp8 small tiles against the dequantising oracle
     (operands e4m3 with fp32 block scales, so only the sums' fp32 rounding
     and the output's bf16 rounding differ)."""
-    counts, n, K = FP8_CASES[i]
+    _check_fp8(ops, *FP8_CASES[i], 200 + i)
+
+
+@pytest.mark.parametrize("i", range(len(FP8_LARGE_CASES)))
+def test_large_fp8_stage_pipeline(ops, i):
+    """The same for the large fp8 tiles, whose fragment reads, scale FMAs and
+    DMAs run across the stage and tile boundaries."""
+    _check_fp8(ops, *FP8_LARGE_CASES[i], 300 + i)
+
+
+def _check_fp8(ops, counts, n, K, seed):
     counts = np.array(counts, np.int64)
     M, E = int(counts.sum()), len(counts)
     offs_h, od = np.cumsum(counts), _offs(counts)
-    rng = np.random.default_rng(200 + i)
+    rng = np.random.default_rng(seed)
     H, N = -(-n // 64) * 64, -(-n // 128) * 128
     x = bf16_dev(rand_bf16(rng, (M, K)))
-    announce(f"small fp8 M={M} E={E} n={n} K={K}")
+    announce(f"fp8 tiles M={M} E={E} n={n} K={K}")
     xq, sx = ops.quantize_fp8_rows(x)
     xd = O.e4m3_bits_to_f32(xq.cpu().numpy()).reshape(M, K // 128, 128) * sx.cpu().numpy().T[:, :, None]
     xd = xd.reshape(M, K)

@@ -20,9 +20,9 @@
 //     scales): one MFMA covers a block's whole k = 128 scale block, and its
 //     partial sum goes straight into the fp32 accumulator times sx * sw, so
 //     the fp32 block scales are applied once per block as in the dequantised
-//     form, with no partial sums kept across MFMAs.  The scale FMAs of token
-//     block jb - 1 run under block jb's MFMAs, and with two waves per SIMD
-//     under the other wave's as well.
+//     form, with no partial sums kept across MFMAs.  A block's scale FMAs run
+//     under the next block's MFMAs, the last block's under the next stage's
+//     first, and with two waves per SIMD under the other wave's as well.
 //   * The 256 x 128 tile was bound by the L2 -> LDS stream (each CU keeps
 //     about 64 line requests in flight), so the tile is as large as the
 //     registers allow: 256 x 256 moves 66 KB per 16.8 MFLOP stage where
@@ -36,12 +36,19 @@
 //     global_load_lds_dwordx4, 8 rows per instruction, XOR-swizzled 16-byte
 //     chunks as in the bf16 kernel), 1 KB of token-row scales (waves 0-3)
 //     and the stage's weight-block scales (waves 4-7 each load a copy, so
-//     every wave issues the same DMA count; all read wave 4's).  At the top
-//     of stage s every wave waits for stage s (the only one in flight) and
-//     passes the barrier, which also means stage s - 1 has been read, and
-//     stage s + 1's weight rows are issued into its buffer (its token rows
-//     and scales after the first token block's MFMAs): one stage ahead
-//     keeps the bounding DMA stream busy.
+//     every wave issues the same DMA count; all read wave 4's).
+//   * The stage barrier sits before a stage's last token block, when the
+//     stage's last fragments are in registers: every wave then waits for
+//     stage s + 1 (the only one in flight), and after the barrier stage
+//     s + 2's weight rows are issued into the buffer of stage s, one DMA
+//     after each MFMA of the last block (its token rows and scales after
+//     those of the next stage's first block).  The next stage's first
+//     fragments are read there too, under the stage's last MFMAs and FMAs.
+//     The DMA stream has no branch but at a tile change: with one in the
+//     loop, the fragments held across the barrier spilled (~150 registers).
+//     Measured against one barrier at the stage's top with the fragment
+//     reads and a DMA burst behind it (DeepSeek-V3 shard, 32768 rows, expert
+//     stage): 1838 -> 1780 us.
 //   * A wave computes only the 16-row token blocks of its half that hold
 //     tile rows (0, 2, 4, 6 or 8, rounded up to even): the k loop is
 //     instantiated per count and picked per tile.  The skipped blocks hold
@@ -49,6 +56,7 @@
 //     stored (short tiles of skewed expert loads).
 //   * Persistent workgroups, XCD-aware slots, flattened (tile, stage) DMA
 //     stream and the EPI_SCATTER metadata in LDS follow gemm_fwd.hip.
+#include <cstdint>
 #include <type_traits>
 
 #include "common.h"
@@ -76,15 +84,18 @@ constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES;   // 132 KB
 constexpr int DMA_P = TP / 8 / WAVES;             // 4
 constexpr int DMA_Q = TQ / 8 / WAVES;             // 4
 static_assert(TQ == 2 * 128 && TP == 4 * 64 && WAVES == 8, "wave layout: 2 token halves x 4 weight quarters");
-// EPI_SCATTER metadata slots (tile round % 3): tile r's slot is written
-// when its first stage is issued, at the top of tile r - 1's last stage,
-// after every wave has passed tile r - 2's epilogue.
+// EPI_SCATTER metadata slots (tile round % 4): tile r's slot is written when
+// the DMA stream reaches its first stage, two stages ahead.  With one stage
+// per tile that is in tile r - 2, before its barrier: every wave has then
+// passed tile r - 4's epilogue, whose slot it is (tile r - 3's may still run).
 constexpr int META_BYTES = TQ * 8;
-constexpr int META_SLOTS = 3;
+constexpr int META_SLOTS = 4;
 constexpr int LDS_TOTAL = LDS_BYTES + META_SLOTS * META_BYTES;  // 138 KB
-static_assert(LDS_TOTAL <= 160 * 1024, "LDS");
+static_assert(NSTAGE == 2 && STAGE_BYTES % 1024 == 0 && LDS_TOTAL <= 160 * 1024, "LDS");
 
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) i32x4_t lds_i32x4_t;
+typedef __attribute__((address_space(3))) int lds_int_t;
 
 // Chunk permutation of 128-byte LDS rows (as in gemm_fwd.hip).
 __device__ __forceinline__ int cswz(int r) { return (r ^ (r >> 3)) & 7; }
@@ -172,35 +183,41 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_kernel(const Fp8Args a) {
     }
     d_r = r;
   };
-  // A stage's weight rows are issued at the barrier that frees their buffer,
-  // its token rows and scales after the first token block's MFMAs (see the
-  // k loop); issue_p sets the stage's bases, which issue_q reads.
-  uint64_t d_sqb = 0;
-  uint32_t d_sst = 0;
-  int d_sks = 0;
-  auto issue_p = [&](int s) {
-    const int r = s / ksteps;
-    const int ks = s - r * ksteps;
-    if (r != d_r) dma_tile(r);
-    const uint64_t pb = d_pbase + (uint64_t)ks * TKB;
-    d_sqb = d_qbase + (uint64_t)ks * TKB;
-    d_sst = lds0 + (uint32_t)((s % NSTAGE) * STAGE_BYTES);
-    d_sks = ks;
-#pragma unroll
-    for (int i = 0; i < DMA_P; ++i) {
-      int prow;  // weight row relative to d_pbase
-      if constexpr (EPI == EPI_SWIGLU)
-        prow = (i < 2) ? min(rr0 + 64 * i, d_hmax) : (int)a.hidden + min(rr0 + 64 * (i - 2), d_hmax);
-      else
-        prow = min(rr0 + 64 * i, d_pmax);
-      dma16((uint32_t)(prow * a.ldp) + lch16, pb, d_sst + w * 1024 + i * (WAVES * 1024));
+  // The DMA stream: advance() steps it to the next stage (past the walk's end
+  // it repeats stages of the last tile, which nothing reads), issue_p and
+  // issue_q load that stage's weight rows, token rows and scales into a
+  // buffer, without a branch.
+  int d_ks = 0;
+  auto advance = [&]() {
+    if (++d_ks == ksteps) {
+      d_ks = 0;
+      if (d_r + 1 < nmy) dma_tile(d_r + 1);
     }
   };
-  auto issue_q = [&]() {
+  auto issue_p = [&](int buf, int i) {
+    int prow;  // weight row relative to d_pbase
+    if constexpr (EPI == EPI_SWIGLU)
+      prow = (i < 2) ? min(rr0 + 64 * i, d_hmax) : (int)a.hidden + min(rr0 + 64 * (i - 2), d_hmax);
+    else
+      prow = min(rr0 + 64 * i, d_pmax);
+    dma16((uint32_t)(prow * a.ldp) + lch16, d_pbase + (uint64_t)d_ks * TKB,
+          lds0 + (uint32_t)(buf * STAGE_BYTES) + w * 1024 + i * (WAVES * 1024));
+  };
+  auto issue_q = [&](int buf, int i) {
+    dma16((uint32_t)(min(rr0 + 64 * i, d_qmax) * a.ldq) + lch16, d_qbase + (uint64_t)d_ks * TKB,
+          lds0 + (uint32_t)(buf * STAGE_BYTES) + P_BYTES + w * 1024 + i * (WAVES * 1024));
+  };
+  auto issue_s = [&](int buf) {
+    dma4(d_scoff, d_scbase + (uint64_t)d_ks * d_scstep, lds0 + (uint32_t)(buf * STAGE_BYTES) + d_sclds);
+  };
+  auto issue_qs = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < DMA_Q; ++i)
-      dma16((uint32_t)(min(rr0 + 64 * i, d_qmax) * a.ldq) + lch16, d_sqb, d_sst + P_BYTES + w * 1024 + i * (WAVES * 1024));
-    dma4(d_scoff, d_scbase + (uint64_t)d_sks * d_scstep, d_sst + d_sclds);
+    for (int i = 0; i < DMA_Q; ++i) issue_q(buf, i);
+    issue_s(buf);
+  };
+  auto issue_ps = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < DMA_P; ++i) issue_p(buf, i);
   };
 
   // ---- fragment geometry -------------------------------------------------------
@@ -213,20 +230,26 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_kernel(const Fp8Args a) {
     arow[pb] = (EPI == EPI_SWIGLU) ? (pb < 2 ? 32 * wp + 16 * pb : 128 + 32 * wp + 16 * (pb - 2))
                                    : 64 * wp + 16 * pb;
   // Row 16m + r16 of a 128-byte-row operand: cswz = f16 ^ ((2m) & 6) (16m >> 3
-  // = 2m is even, so adding r16 >> 3 does not carry).
-  auto frag16 = [&](const char* base, int row0) {
-    const int x = f16 ^ ((row0 >> 3) & 6);
-    const char* row = base + (row0 + r16) * TKB;
-    const i32x4_t lo = *(const i32x4_t*)(row + (((2 * g4) ^ x) * 16));
-    const i32x4_t hi = *(const i32x4_t*)(row + (((2 * g4 + 1) ^ x) * 16));
-    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  // = 2m is even, so adding r16 >> 3 does not carry).  The stage buffers are
+  // aligned to 1 KB, so a row block's permutation is an XOR on the lane's
+  // address in the buffer (fv), which is all that is kept in registers.
+  const uint32_t fv = lds0 + r16 * TKB + (uint32_t)(((2 * g4) ^ f16) * 16);
+  auto frag16 = [&](uint32_t st, int off, int row0) {
+    const uint32_t lo = ((fv + st) ^ (uint32_t)(((row0 >> 3) & 6) * 16)) + off + row0 * TKB;
+    const i32x4_t vlo = *(const lds_i32x4_t*)(uintptr_t)lo;
+    const i32x4_t vhi = *(const lds_i32x4_t*)(uintptr_t)(lo ^ 16);
+    return __builtin_shufflevector(vlo, vhi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
   // weight-block scale of block pb (the copy wave 4 loaded)
   auto sw_lane = [&](int pb) { return (EPI == EPI_SWIGLU) ? (pb < 2 ? 0 : 1 + wp) : (wp >> 1); };
 
-  // ---- prologue: stage 0 in flight ----------------------------------------------
-  issue_p(0);
-  issue_q();
+  // ---- prologue: stage 0 has landed, stage 1 in flight ---------------------------
+  dma_tile(0);
+  issue_ps(0);
+  issue_qs(0);
+  wait_vm_barrier<0>();
+  advance();
+  issue_ps(1);
 
   int s = 0;
   for (int r = 0; r < nmy; ++r) {
@@ -251,46 +274,65 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_kernel(const Fp8Args a) {
     const int nbw = (((hq + 15) >> 4) + 1) & ~1;
     auto kloop = [&](auto nbc) {
       constexpr int NB = decltype(nbc)::value;
-      for (int ks = 0; ks < ksteps; ++ks, ++s) {
-        // Stage s has landed (the only stage in flight) and every wave is
-        // done with stage s - 1: its buffer takes stage s + 1.  The DMA
-        // stream is the bound, so one stage ahead keeps it busy.
-        wait_vm_barrier<0>();
-        const bool more = s + 1 < total;
-        if (more) issue_p(s + 1);
-        if constexpr (NB == 0) {
-          if (more) issue_q();
-        } else {
-          const char* st = smem + (s % NSTAGE) * STAGE_BYTES;
-          i32x8_t fa[NPB16];
-          // A block's weight scale is one value for the whole wave (every lane
-          // reads the same LDS word): kept in SGPRs, it frees VGPRs for the
-          // accumulators and fragments.
-          float swv[NPB16];
+      // The stage barrier: stage s + 1 has landed (the only stage in flight)
+      // and every wave has read all of stage s, whose buffer takes stage
+      // s + 2.  Every wave passes exactly one per stage.
+      if constexpr (NB == 0) {
+        for (int ks = 0; ks < ksteps; ++ks, ++s) {
+          issue_qs((s + 1) & 1);
+          advance();
+          wait_vm_barrier<0>();
+          issue_ps(s & 1);
+        }
+      } else {
+        i32x8_t fa[NPB16];
+        i32x8_t fb[NBS];
+        float sxv[NBS];
+        // A block's weight scale is one value for the whole wave (every lane
+        // reads the same LDS word): kept in SGPRs, it frees VGPRs for the
+        // accumulators and fragments.
+        int swr[NPB16];
+        float swv[NPB16];
+        auto read_a = [&](uint32_t st, int pb) {
+          fa[pb] = frag16(st, 0, arow[pb]);
+          swr[pb] = *(const lds_int_t*)(uintptr_t)(lds0 + st + SW_OFF + sw_lane(pb) * 4);
+        };
+        auto read_b = [&](uint32_t st, int jb) {
+          const int row = 128 * wq + 16 * jb;
+          fb[jb % NBS] = frag16(st, P_BYTES, row);
+          sxv[jb % NBS] = __int_as_float(*(const lds_int_t*)(uintptr_t)(lds0 + st + SX_OFF + (row + r16) * 4));
+        };
+        auto take_sw = [&]() {
 #pragma unroll
-          for (int pb = 0; pb < NPB16; ++pb) {
-            fa[pb] = frag16(st, arow[pb]);
-            swv[pb] = __int_as_float(__builtin_amdgcn_readfirstlane(*(const int*)(st + SW_OFF + sw_lane(pb) * 4)));
-          }
-          i32x8_t fb[NBS];
-          float sxv[NBS];
-          auto read_b = [&](int jb) {
-            const int row = 128 * wq + 16 * jb;
-            fb[jb % NBS] = frag16(st + P_BYTES, row);
-            sxv[jb % NBS] = *(const float*)(st + SX_OFF + (row + r16) * 4);
-          };
-          read_b(0);
-          read_b(1);
-          float sx_prev = 0.f;
-          floatx4_t part[2][NPB16];
-          auto scale_add = [&](int jb, float sxj) {
+          for (int pb = 0; pb < NPB16; ++pb) swv[pb] = __int_as_float(__builtin_amdgcn_readfirstlane(swr[pb]));
+        };
+        {
+          const uint32_t st = (s & 1) * STAGE_BYTES;
 #pragma unroll
-            for (int pb = 0; pb < NPB16; ++pb) {
-              const float sc = swv[pb] * sxj;
+          for (int pb = 0; pb < NPB16; ++pb) read_a(st, pb);
+          read_b(st, 0);
+          read_b(st, 1);
+        }
+        take_sw();
+        // A block's scale FMAs run under the next block's MFMAs, the stage's
+        // last block's under the next stage's first.
+        floatx4_t part[2][NPB16];
+        float sx_prev = 0.f;
+        float swp[NPB16];
 #pragma unroll
-              for (int v = 0; v < 4; ++v) acc[pb][jb][v] += part[jb & 1][pb][v] * sc;
-            }
-          };
+        for (int pb = 0; pb < NPB16; ++pb) {
+          swp[pb] = 0.f;
+          part[1][pb] = floatx4_t{};
+        }
+        auto scale_add = [&](int jb, int pb, float swb) {
+          const float sc = swb * sx_prev;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[pb][jb][v] += part[jb & 1][pb][v] * sc;
+        };
+        for (int ks = 0; ks < ksteps; ++ks, ++s) {
+          const uint32_t st = (s & 1) * STAGE_BYTES;
+          // (past a tile's last stage the reads from stn are in bounds and unused)
+          const uint32_t stn = ((s + 1) & 1) * STAGE_BYTES;
 #pragma unroll
           for (int jb = 0; jb < NB; ++jb) {
 #pragma unroll
@@ -300,16 +342,40 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_kernel(const Fp8Args a) {
               // v_mfma_f32_16x16x128_f8f6f4; the scaled form with unit E8M0
               // scales (127) gives bit-identical sums and runs 2-3 % slower here.
               part[jb & 1][pb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fa[pb], fb[jb % NBS], z, 0, 0, 0, 0, 0, 0);
+              if (jb == 0) {
+                issue_q((s + 1) & 1, pb);
+                if (pb == NPB16 - 1) issue_s((s + 1) & 1);
+              }
+              if (jb == NB - 1) issue_p(s & 1, pb);
+              scale_add(jb > 0 ? jb - 1 : NB - 1, pb, jb > 0 ? swv[pb] : swp[pb]);
+              __builtin_amdgcn_sched_barrier(0);
             }
-            // block jb - 1's scale FMAs run under block jb's MFMAs; block jb's
-            // slot then takes block jb + 2, so its row scale is kept aside first
-            if (jb > 0) scale_add(jb - 1, sx_prev);
+            if (jb == NB - 1) {  // the weight fragments' last use
+#pragma unroll
+              for (int pb = 0; pb < NPB16; ++pb) read_a(stn, pb);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+            // block jb's slot takes block jb + 2, so its row scale is kept aside
             sx_prev = sxv[jb % NBS];
-            if (jb + 2 < NB) read_b(jb + 2);
-            if (jb == 0 && more) issue_q();  // (later placements spill)
+            if (jb == 0) advance();
+            if (jb == NB - 2) {
+              // The stage's last fragments are in registers: turn to the next
+              // stage here, so that its first fragments are read under this
+              // stage's last MFMAs and scale FMAs.
+              wait_vm_barrier<0>();
+            }
+            if (jb + 2 < NB)
+              read_b(st, jb + 2);
+            else
+              read_b(stn, jb + 2 - NB);
+            if (jb >= NB - 2) __builtin_amdgcn_sched_barrier(0);
           }
-          scale_add(NB - 1, sx_prev);
+#pragma unroll
+          for (int pb = 0; pb < NPB16; ++pb) swp[pb] = swv[pb];
+          take_sw();
         }
+#pragma unroll
+        for (int pb = 0; pb < NPB16; ++pb) scale_add(NB - 1, pb, swp[pb]);
       }
     };
     switch (nbw) {
