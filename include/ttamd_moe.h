@@ -12,6 +12,11 @@
  * done on the host before anything is launched, so a rejected call launches
  * nothing.
  *
+ * The ttamd_*workspace_bytes and ttamd_gemm_plan_bytes queries never return
+ * less for more rows, tokens or experts (all else equal), so a workspace or
+ * plan sized for a caller's largest batch serves every smaller one.  (A plan's
+ * contents belong to the rows it was built for.)
+ *
  * bf16 tensors are raw 16-bit brain-float bits, row-major.  Routed rows are
  * numbered j = 0..M-1 with M = num_tokens * topk; "flat" slot s = t*topk + k
  * is the k-th expert choice of token t (the order of
@@ -333,8 +338,9 @@ int ttamd_moe_group_labels(const int32_t* counts_group, int num_groups,
 size_t ttamd_gemm_workspace_bytes(int64_t num_rows, int num_experts);
 
 /* Bytes of a tile plan (gemm_plan of ttamd_router_route and
- * ttamd_moe_experts_forward): the token-tile table of num_rows
- * expert-sorted rows and the split-tile arrival counters.  No counterpart
+ * ttamd_moe_experts_forward): the token-tile tables of num_rows
+ * expert-sorted rows (large and small tiles) and the split-tile arrival
+ * counters.  No counterpart
  * in the reference, whose grouped GEMM plans inside the operator. */
 size_t ttamd_gemm_plan_bytes(int64_t num_rows, int num_experts);
 

@@ -158,3 +158,37 @@ def test_route_noalloc_rejects_oversize_and_bad_arguments():
     assert "sorted_scores" in msg
     msg = _err(lib.ttamd_moe_route_noalloc(None, 1, 8, 4, None, None, None, p, None, None, None))
     assert "null" in msg
+
+
+def _never_smaller(sizes):
+    return [i for i in range(1, len(sizes)) if sizes[i] < sizes[i - 1]]
+
+
+@pytest.mark.parametrize("E", [1, 8, 32, 128, 256, 1024])
+def test_gemm_workspace_sized_for_the_largest_batch_serves_smaller_ones(E):
+    """Workspaces and plans never shrink with more rows (or experts): a caller
+    that sizes them once for its largest batch is not refused on a smaller
+    one.  Row counts around every line of the small-tile rule included."""
+    lib = _lib.load()
+    rows = sorted({*range(0, 20000, 7), *(b + d for b in (768, 32 * E + 31, 100 * E, 8192) for d in (-1, 0, 1)),
+                   1 << 17, 1 << 20, 1 << 28})
+    for fn in (lib.ttamd_gemm_plan_bytes, lib.ttamd_gemm_workspace_bytes,
+               lambda m, e: lib.ttamd_router_backward_workspace_bytes(m, min(e, 256), 2048),
+               lambda m, e: lib.ttamd_moe_experts_forward_workspace_bytes(m, 2048, 768, e, 1, 0)):
+        assert not _never_smaller([fn(m, E) for m in rows])
+        assert all(fn(m, E) >= fn(m, max(1, E // 2)) for m in rows)
+
+
+@pytest.mark.parametrize("E", [6, 128, 256])
+def test_router_workspace_sized_for_the_largest_batch_serves_smaller_ones(E):
+    """The same for the router's partial logits, over token counts (few tokens
+    are cut into more slices of D, many into fewer) and over D."""
+    lib = _lib.load()
+    tokens = sorted({*range(1, 3000, 3), *range(3000, 70000, 61), *(128 * n + d for n in (1, 2, 85, 86, 128, 255, 256)
+                                                                 for d in (0, 1))})
+    dims = [64, 128, 192, 256, 512, 1024, 2048, 2112, 4096, 5120, 7168]
+    for fn in (lib.ttamd_router_workspace_bytes, lambda t, e, d: lib.ttamd_router_route_workspace_bytes(t, e, d, 4)):
+        for d in dims:
+            assert not _never_smaller([fn(t, E, d) for t in tokens]), d
+        for t in (1, 128, 256, 257, 8192, 65536):
+            assert not _never_smaller([fn(t, E, d) for d in dims]), t

@@ -53,9 +53,10 @@ int gemm_fwd_tile_rows() { return kFwdTileRows; }
 static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // The tile plan: header, split-tile counters, tile table, small-tile table.
+// Never smaller for more rows or experts.
 size_t gemm_plan_bytes(int64_t M, int E) {
   return sizeof(int4) + kSplitTiles * sizeof(int) +
-         (size_t)(max_row_tiles((int)M, E) + max_small_tiles((int)M, E)) * sizeof(int4) + 256;
+         (size_t)(max_row_tiles((int)M, E) + small_table_tiles(M, E)) * sizeof(int4) + 256;
 }
 
 // Partial sums of the split leftover tiles: one piece per workgroup at most.

@@ -1,6 +1,8 @@
 // Pieces shared by the grouped GEMM kernels (internal to libttamd_moe.so).
 #pragma once
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace ttamd {
@@ -37,8 +39,9 @@ constexpr int kFwdTileRows = 320;
 // Tile plan of a token-row GEMM: int4 header {number of tiles, number of
 // small tiles, ...}, the arrival counters of the split tail tiles
 // (kSplitTiles ints, zeroed whenever a table is built and left at zero by
-// every GEMM that uses them), the tile table, then (small_tile_rows(M, E) >
-// 0) the table of the small-tile kernel.
+// every GEMM that uses them), the tile table, then the table of the
+// small-tile kernel (filled where small_tile_rows(M, E) > 0; the room for it
+// is there for every M).
 constexpr int kSplitTiles = 512;
 struct TileTable {
   int* count;
@@ -60,14 +63,21 @@ inline int max_row_tiles(int M, int E) { return M / kTileRows + E + 1; }
 // tiles are ahead, 42 against 50 us on 4 experts of 2048 x 1024).
 constexpr int kSmallAvgRows = 100;
 constexpr int kSmallMaxRows = 8192;
+inline int64_t small_rows64_max(int E) { return std::max<int64_t>(32 * (int64_t)E + 31, 768); }
+inline int64_t small_rows128_max(int E) { return std::max<int64_t>(kSmallAvgRows * (int64_t)E, kSmallMaxRows); }
 inline int small_tile_rows(int M, int E) {
-  if (M <= 32 * (int64_t)E + 31 || M <= 768) return 64;
-  return M <= kSmallAvgRows * (int64_t)E || M <= kSmallMaxRows ? 128 : 0;
+  if (M <= small_rows64_max(E)) return 64;
+  return M <= small_rows128_max(E) ? 128 : 0;
 }
 // An expert's c rows make at most ceil(c / rows) tiles.
 inline int max_small_tiles(int M, int E) {
   const int rows = small_tile_rows(M, E);
   return rows > 0 ? M / rows + E + 1 : 0;
+}
+// The most small tiles of any call of at most M rows: what a plan has room
+// for, so that one sized for the largest batch serves every smaller one.
+inline int64_t small_table_tiles(int64_t M, int E) {
+  return std::max(std::min(M, small_rows64_max(E)) / 64, std::min(M, small_rows128_max(E)) / 128) + E + 1;
 }
 
 inline TileTable tile_table_in(void* ws, int M, int E) {

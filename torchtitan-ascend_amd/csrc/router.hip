@@ -529,21 +529,33 @@ hipError_t launch_gemm_eb(const RouterGemmArgs& a, int S, hipStream_t stream) {
 // partials are small and a slice's length is what a call waits for: up to
 // kRouterFewSplits slices of at least 2 stages (32 tokens, D = 2048, E = 128:
 // 8.5 -> 5.2 us).
+constexpr int kRouterFewTiles = 2;
+int router_few_cap(int stages) { return max(1, min(kRouterFewSplits, stages / 2)); }
+int router_cap(int stages) { return max(1, min(kRouterMaxSplits, stages / 4)); }
 int router_splits(int T, int D) {
   const int tiles = (T + RT - 1) / RT;
   const int stages = D / RTK;
-  int S = (num_cus() + tiles - 1) / tiles;
-  S = tiles <= 2 ? min(min(S, kRouterFewSplits), stages / 2) : min(min(S, kRouterMaxSplits), stages / 4);
-  S = max(1, S);
+  const int S = min((num_cus() + tiles - 1) / tiles, tiles <= kRouterFewTiles ? router_few_cap(stages) : router_cap(stages));
   const int per = (stages + S - 1) / S;
   return (stages + per - 1) / per;  // no empty slice
 }
 
 }  // namespace
 
+// The most partial logits that any call of at most T tokens and D columns
+// writes, not only this T's: a workspace sized for the largest batch then
+// serves every smaller one, whose calls may cut D into more slices.
 size_t router_workspace_bytes(int64_t T, int E, int64_t D) {
   if (T <= 0) return 0;
-  return (size_t)router_splits((int)T, (int)D) * (size_t)T * (size_t)E * sizeof(float) + 256;
+  const int stages = (int)(D / RTK), cus = num_cus();
+  const int64_t tiles = (T + RT - 1) / RT;
+  int64_t rows = std::min<int64_t>(T, kRouterFewTiles * RT) * std::min(cus, router_few_cap(stages));
+  for (int S = 1; S <= router_cap(stages); ++S) {
+    // n tiles are cut into S slices or more up to ceil(CUs / n) >= S
+    const int64_t n = S == 1 ? tiles : std::min<int64_t>(tiles, (cus - 1) / (S - 1));
+    rows = std::max(rows, std::min(T, n * RT) * S);
+  }
+  return (size_t)rows * (size_t)E * sizeof(float) + 256;
 }
 
 hipError_t launch_router_fused(const void* x, const void* w, const float* bias, int T, int E, int D, int K,
