@@ -344,6 +344,18 @@ size_t ttamd_gemm_workspace_bytes(int64_t num_rows, int num_experts);
  * in the reference, whose grouped GEMM plans inside the operator. */
 size_t ttamd_gemm_plan_bytes(int64_t num_rows, int num_experts);
 
+/* Which tiles a forward grouped GEMM of this library runs on, for reports
+ * and tests (nothing is launched): host_counts is a HOST array of the rows
+ * per expert, weight_rows the weight rows per expert (2 H for the SwiGLU
+ * GEMMs), fp8 nonzero for the fp8 GEMMs.  *tile_rows x *tile_cols: token rows
+ * at most x weight rows of a tile (320 x 256 and, in fp8, 256 x 256: the large
+ * kernels; 64 or 128 x 128 or 256: the small-tile ones); *split_pieces:
+ * pieces that each tile left over after the last full round is cut into
+ * (1: none).  No counterpart in the reference. */
+int ttamd_gemm_tiles(const int32_t* host_counts, int num_experts,
+                     int64_t weight_rows, int64_t k, int fp8, int* tile_rows,
+                     int* tile_cols, int* split_pieces);
+
 /*
  * out[m, n] = sum_k x[m, k] * w[e(m), n, k]  (bf16 out).
  * Replaces torch._grouped_mm(x, w.transpose(-2,-1), offs)

@@ -192,3 +192,28 @@ def test_router_workspace_sized_for_the_largest_batch_serves_smaller_ones(E):
             assert not _never_smaller([fn(t, E, d) for t in tokens]), d
         for t in (1, 128, 256, 257, 8192, 65536):
             assert not _never_smaller([fn(t, E, d) for d in dims]), t
+
+
+def _tiles(*args):
+    return importlib.import_module("torchtitan-ascend_amd.ops").gemm_tiles(*args)
+
+
+@pytest.mark.parametrize("counts,weight_rows,k,large", [
+    # one expert with a long reduction and few tiles (a shared expert's w2):
+    # the large tiles' tail split fills the chip
+    ((8,), 5120, 8192, True), ((64,), 5120, 8192, True), ((128,), 5120, 8192, True), ((800,), 5120, 8192, True),
+    ((4000,), 5120, 8192, True),     ((320,), 16384, 5120, True),
+    # tiles of less than 320 rows cost less than one of 320
+    ((375,) * 4, 7168, 2048, True), ((5000,), 2048, 4096, True),
+    # the same experts where the small tiles are ahead
+    ((64,), 16384, 5120, False), ((320,), 5120, 8192, False), ((640,), 5120, 8192, False), ((200,), 7168, 2048, False), ((1500,), 2048, 4096, False),
+    ((500,), 1536, 2048, False), ((256,) * 8, 1024, 256, False), ((2,) * 128, 1536, 2048, False),
+    ((63,) * 128, 2048, 768, False), ((7,) * 28 + (0,) * 4, 4096, 7168, False), ((88,) * 32, 7168, 2048, False),
+    # prefill and training loads
+    ((512,) * 128, 1536, 2048, True), ((8192,), 16384, 5120, True), ((128,) * 16, 5120, 8192, True),
+])
+def test_gemm_tile_choice(counts, weight_rows, k, large):
+    """Each shape on the tiles that were measured ahead on it (times beside
+    the rule, small_tile_cols)."""
+    rows, cols, _ = _tiles(counts, weight_rows, k)
+    assert (rows == 320) == large, (rows, cols)

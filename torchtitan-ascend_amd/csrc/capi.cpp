@@ -538,6 +538,23 @@ size_t ttamd_gemm_plan_bytes(int64_t num_rows, int num_experts) {
   return ttamd::gemm_plan_bytes(num_rows, num_experts);
 }
 
+int ttamd_gemm_tiles(const int32_t* host_counts, int num_experts, int64_t weight_rows, int64_t k, int fp8,
+                     int* tile_rows, int* tile_cols, int* split_pieces) {
+  const char* fn = "ttamd_gemm_tiles";
+  REQUIRE(host_counts && tile_rows && tile_cols && split_pieces, "%s: null pointer argument", fn);
+  REQUIRE(num_experts >= 1 && num_experts <= 1024, "%s: num_experts must be in [1, 1024] (got %d)", fn, num_experts);
+  int64_t rows = 0;
+  for (int e = 0; e < num_experts; ++e) {
+    REQUIRE(host_counts[e] >= 0, "%s: negative count", fn);
+    rows += host_counts[e];
+  }
+  REQUIRE(rows <= (1 << 28), "%s: num_rows out of range (%lld)", fn, (long long)rows);
+  TRY(check_dim(fn, "weight_rows", weight_rows, 128));
+  TRY(check_dim(fn, "k", k, fp8 ? 128 : 64));
+  ttamd::gemm_tiles(host_counts, num_experts, weight_rows, (int)k, fp8 != 0, tile_rows, tile_cols, split_pieces);
+  return TTAMD_OK;
+}
+
 int ttamd_grouped_mm(const void* x, const void* w, const int32_t* offs, int64_t num_rows,
                      int num_experts, int64_t n, int64_t k, void* out, void* workspace,
                      size_t workspace_bytes, void* stream) {

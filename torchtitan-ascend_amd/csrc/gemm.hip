@@ -86,31 +86,84 @@ void probe_chain_arm(const hipEvent_t* events, int n_launches) {
   p.chain_n = n_launches > 0 ? n_launches : 0;
 }
 
-// Weight rows per tile if a forward GEMM over `cols` weight rows per expert
-// takes the small-tile kernel, 0 if the large one (large_rows x 256: 320 rows
-// in bf16, 256 in fp8).
+// Token tiles of at most h rows that M rows over E experts make, near-even
+// loads: every hit expert's share of the rows in whole tiles, or, with fewer
+// rows than a tile each, the row count with a partial tile for every third.
+static int64_t expected_qtiles(int M, int E, int h) {
+  const int64_t hit = std::max(1, std::min(E, M));
+  return std::max<int64_t>(hit * ((M + h * hit - 1) / (h * hit)), (M + h - 1) / h + (hit - 1) / 3);
+}
+static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Weight rows per tile if a bf16 forward GEMM over `cols` weight rows of k
+// columns per expert takes the small-tile kernel, 0 if the large one (320 x
+// 256).
 //
-// Up to kSmallAvgRows rows per expert on average the GEMM streams weights
-// and the small tiles' deeper ring is ahead (Qwen3-30B-A3B experts, both
-// GEMMs and the K-way sum: 2 rows 243 -> 196 us, 21 rows 283 -> 230, 63
-// rows 299 -> 251, 96 rows 315 -> 281; DeepSeek-V3's 94 rows 632 -> 530); at
-// 125-128 rows many experts need a second 128-row tile and it is not (331 ->
-// 337 us, 664 -> 680 us).  With more rows per expert it pays where the large
-// tiles leave the chip idle in their last round and the weights are re-read
-// from the memory-side cache (256 MB): the rounds of each tiling are weighed
-// with its time per 64-k stage (measured on whole rounds: 2.0 us for 320 x
-// 256, 1.08 for 128 x 256, 0.66 for 128 x 128, 0.85 for 64 x 256 and 0.5 for
-// 64 x 128), e.g. 4 experts of 2048 x 1024 with 2000 rows 98 -> 57 us, with
-// 8000 rows 121 us against 133 (kept large).  Weights that stream from HBM
-// or two and more rounds of large tiles are better left alone (Llama4-Scout
-// w2, 128 rows per expert: 348 us against 388; w13 568 against 664).
+// Up to kSmallAvgRows rows per expert on average the GEMM streams weights.
+// Measured on w13 / w2, us, small against large: 128 experts of 768 x 2048
+// with an even load, 2 rows each 127 / 66 against 129 / 69, 40 rows 152 / 89
+// against 147 / 88, 100 rows 171 / 104 against 160 / 103; with a Zipf(0.8)
+// load 72 rows 173 / 100 against 218 / 103; 32 experts of 7168 x 2048, 9 rows
+// 306 / 166 against 307 / 179, 88 rows 324 / 195 against 326 / 195, Zipf(1.2)
+// 72 rows 381 / 199 against 319 / 194.  So an even load is about a tie, the
+// small tiles are ahead where few long segments leave the large ones ragged,
+// and behind where their own tiles just pass a round; the load is not known
+// here, and they stay.  At 128 rows many experts need a second 128-row tile
+// (even 207 / 117 against 164 / 108) and the large ones are taken.
+//
+// With more rows per expert the small tiles pay where the large ones leave
+// the chip idle in their last round and the weights are re-read from the
+// memory-side cache (256 MB): the rounds of each tiling are weighed with its
+// time per 64-k stage (0.01 us, 320 x 256: 200, 128 x 256: 108, 128 x 128: 66,
+// 64 x 256: 85, 64 x 128: 50); weights that stream from HBM or two and more
+// rounds of large tiles are left alone.
+//
+// In both cases the large tiles may be ahead all the same: by their tail
+// split (a reduction cut over workgroups that would idle) and where their
+// tiles have less than 320 rows.  Both sides are therefore estimated in time
+// (fixed cost per tile, time per stage, the weights' stream; for the split
+// its share of the stages and the partial sums), with constants from runs of
+// 1 to 4 experts of 5120 x 8192, 16384 x 5120, 7168 x 2048, 2048 x 4096, 2048
+// x 768 and 1536 x 2048 with 8 to 8192 rows, and the small ones dropped where
+// they lose by 7 %.  One expert, large against small: 5120 x 8192, 8 rows 33
+// against 44 us, 64 rows 38 against 53, 800 rows 94 against 109, 4000 rows
+// 272 against 368; 16384 x 5120, 320 rows 86 against 100; small ahead: 5120 x
+// 8192, 320 rows 59 against 91, 16384 x 5120, 64 rows 37 against 43, 1536 x
+// 2048, 500 rows 17 against 48.
 constexpr int64_t kSmallWeightBytes = 256 << 20;
-static int small_tile_cols(int M, int E, int64_t cols, int64_t row_bytes, int large_rows) {
+static int small_tile_cols(int M, int E, int64_t cols, int k) {
+  const int rows = small_tile_rows(M, E);
+  if (rows == 0) return 0;
+  const int64_t G = (num_cus() + 7) & ~7, stages = k / 64;
+  const int64_t large_q = expected_qtiles(M, E, kFwdTileRows), large_tiles = large_q * ceil_div(cols, 256);
+  const int64_t weights = std::min(E, M) * cols * k * 2;
+  auto rounds = [&](int c) { return ceil_div(expected_qtiles(M, E, rows) * ceil_div(cols, c), G); };
+  const int64_t c128 = rounds(128) * (rows == 64 ? 50 : 66), c256 = rounds(256) * (rows == 64 ? 85 : 108);
+  const int small = c128 < c256 ? 128 : 256;
+  const bool few_rows = M <= kSmallAvgRows * (int64_t)E;
+  if (few_rows && large_tiles >= G) return small;
+  if (!few_rows && (weights > kSmallWeightBytes || large_tiles >= 2 * G ||
+                    std::min(c128, c256) >= ceil_div(large_tiles, G) * 200))
+    return 0;
+  // 0.01 us
+  const int64_t stream = weights / (weights > kSmallWeightBytes ? 60000 : 130000);
+  const int64_t small_time = std::min(rounds(128) * (rows == 64 ? 160 + (M <= 32 * (int64_t)E ? 29 : 37) * stages : 230 + 55 * stages),
+                                      rounds(256) * (rows == 64 ? 160 + 60 * stages
+                                                                : 450 + (rounds(256) > 1 ? 93 : 83) * stages));
+  const int64_t h = std::min<int64_t>(kFwdTileRows, (ceil_div(M, large_q) + 31) & ~31);
+  const int64_t fixed = 100 + 23 * h / 10, work = stages * std::max<int64_t>(107, 150 * h / 256);
+  const int64_t R = large_tiles / G, rt = large_tiles - R * G;
+  const int np = split_pieces((int)R, (int)rt, (int)G, (int)stages, split_max());
+  // partial sums of a split: cheaper with few leftover tiles
+  const int64_t partials = h * (50 + 12 * np) * std::min<int64_t>(std::max<int64_t>(rt, 6), 20) / 200 + 300;
+  const int64_t large_time = np > 1 ? R * (fixed + work) + fixed + work / np + partials : (R + (rt > 0)) * (fixed + work);
+  return 100 * (600 + std::max(small_time, stream)) > 107 * (600 + std::max(large_time, stream * 105 / 100)) ? 0 : small;
+}
+
+static int fp8_small_cols(int M, int E, int64_t cols, int64_t row_bytes) {
   const int rows = small_tile_rows(M, E);
   if (rows == 0) return 0;
   const int64_t G = (num_cus() + 7) & ~7;
-  // token tiles of at most h rows: one per hit expert, or by the row count
-  // with a partial tile for every third expert
   auto qtiles = [&](int h) {
     const int64_t hit = std::min(E, M);
     return std::max<int64_t>(hit, (M + h - 1) / h + (hit - 1) / 3);
@@ -120,10 +173,27 @@ static int small_tile_cols(int M, int E, int64_t cols, int64_t row_bytes, int la
   const int64_t c128 = cost(rows, 128, rows == 64 ? 50 : 66), c256 = cost(rows, 256, rows == 64 ? 85 : 108);
   const int small = c128 < c256 ? 128 : 256;
   if (M <= kSmallAvgRows * (int64_t)E) return small;
-  return std::min(E, M) * cols * row_bytes <= kSmallWeightBytes && tiles(large_rows, 256) < 2 * G &&
-                 std::min(c128, c256) < cost(large_rows, 256, 200)
+  return std::min(E, M) * cols * row_bytes <= kSmallWeightBytes && tiles(kFp8TileRows, 256) < 2 * G &&
+                 std::min(c128, c256) < cost(kFp8TileRows, 256, 200)
              ? small
              : 0;
+}
+
+// The tiles a forward GEMM with these host counts runs on (ttamd_gemm_tiles).
+void gemm_tiles(const int* counts, int E, int64_t weight_rows, int k, bool fp8, int* tile_rows, int* tile_cols,
+                int* pieces) {
+  int64_t M = 0;
+  for (int e = 0; e < E; ++e) M += counts[e];
+  const int small = fp8 ? fp8_small_cols((int)M, E, weight_rows, k) : small_tile_cols((int)M, E, weight_rows, k);
+  *tile_rows = small ? small_tile_rows((int)M, E) : fp8 ? kFp8TileRows : kFwdTileRows;
+  *tile_cols = small ? small : 256;
+  *pieces = 1;
+  if (small || fp8) return;
+  int64_t tiles = 0;
+  for (int e = 0; e < E; ++e) tiles += tiles_of(counts[e], kFwdTileRows);
+  tiles *= ceil_div(weight_rows, 256);
+  const int64_t G = (num_cus() + 7) & ~7;
+  if (tiles / G <= kSplitMaxRounds) *pieces = split_pieces((int)(tiles / G), (int)(tiles % G), (int)G, k / 64, split_max());
 }
 
 // plan: the tile plan; part: the partial-sum area of split leftover tiles
@@ -136,7 +206,7 @@ static hipError_t fwd(int epi, FwdGemm g, const int* offs, int E, int M, void* p
     if (err != hipSuccess) return err;
   }
   const TileTable tt = tile_table_in(plan, M, E);
-  const int small = small_tile_cols(M, E, epi == EPI_SWIGLU ? 2 * (int64_t)g.n : g.n, 2 * (int64_t)g.kred, kFwdTileRows);
+  const int small = small_tile_cols(M, E, epi == EPI_SWIGLU ? 2 * (int64_t)g.n : g.n, g.kred);
   g.table = small ? tt.small_table : tt.table;
   g.n_qtiles = small ? tt.small_count : tt.count;
   g.split_cnt = tt.split_cnt;
@@ -249,7 +319,7 @@ static hipError_t fp8(int epi, Fp8Args a, const int* offs, int E, int M, void* w
   hipError_t err = launch_tile_map(offs, E, M, kFp8TileRows, ws, true, stream);
   if (err != hipSuccess) return err;
   const TileTable tt = tile_table_in(ws, M, E);
-  const int small = small_tile_cols(M, E, a.n_p, a.kred, kFp8TileRows);
+  const int small = fp8_small_cols(M, E, a.n_p, a.kred);
   a.table = small ? tt.small_table : tt.table;
   a.n_qtiles = small ? tt.small_count : tt.count;
   return small ? launch_small_fp8_gemm(epi, a, tt.small_rows, small, stream) : launch_fp8_gemm(epi, a, stream);

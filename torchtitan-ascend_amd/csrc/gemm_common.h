@@ -106,6 +106,22 @@ constexpr size_t kSplitPartBytes = 327680;  // 8 waves x 160 fp32 x 64 lanes
 constexpr int kSplitMaxPieces = 8;
 constexpr int kSplitMinStages = 8;
 constexpr int kSplitMaxRounds = 6;
+// Pieces per leftover tile of a walk of R full rounds of G workgroups and rt
+// leftover tiles (1: no split).  The last piece reads every partial, so at
+// most sqrt(ksteps / 2) pieces, and two only for long reductions.
+__host__ __device__ inline int split_pieces(int R, int rt, int G, int ksteps, int most) {
+  if (rt <= 0 || rt > kSplitTiles || R > kSplitMaxRounds) return 1;
+  int np = std::max(1, std::min(std::min(G / rt, most), ksteps / kSplitMinStages));
+  while (np > 1 && ksteps < 2 * np * np) --np;
+  return np == 2 && ksteps < 64 ? 1 : np;
+}
+
+// Height of the tiles of an expert's c > 0 rows, and their number.
+__host__ __device__ inline int tile_height(int c, int max_rows) {
+  const int n = (c + max_rows - 1) / max_rows;
+  return (((c + n - 1) / n) + 31) & ~31;
+}
+inline int tiles_of(int c, int max_rows) { return c > 0 ? (c + tile_height(c, max_rows) - 1) / tile_height(c, max_rows) : 0; }
 
 // Builds one tile table with one workgroup of NT threads (every thread
 // calls it; it synchronises the workgroup).  `range(e, r0, r1)` gives the
@@ -128,8 +144,7 @@ __device__ void block_tile_table(Range range, int E, int max_tiles, int max_rows
       range(e, r0, r1);
       const int c = r1 - r0;
       if (c > 0) {
-        const int n0 = (c + max_rows - 1) / max_rows;
-        h = (((c + n0 - 1) / n0) + 31) & ~31;
+        h = tile_height(c, max_rows);
         nt = (c + h - 1) / h;
       }
     }
@@ -319,6 +334,8 @@ hipError_t launch_tile_map(const int* offs, int E, int M, int max_rows, void* ws
 // weight rows per tile (gemm_small.hip).
 hipError_t launch_fwd_gemm(int epi, const FwdGemm& g, int small_rows, int small_cols, hipStream_t stream);
 hipError_t launch_small_gemm(int epi, FwdArgs a, int tile_rows, int tile_cols, hipStream_t stream);
+// Most pieces of a split leftover tile.
+int split_max();
 // dgrad GEMM (EPI_STORE or EPI_SWIGLU_BWD) over the same tile table.
 hipError_t launch_dgrad_gemm(int epi, const DgradGemm& g, hipStream_t stream);
 // fp8 forward GEMM over a tile table of at most kFp8TileRows rows per tile.

@@ -162,15 +162,7 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
   // every slot runs R whole tiles, then at most one piece.
   const int R = U(ntiles / G);
   const int rt = ntiles - R * G;
-  int np = 1;
-  if (a.part != nullptr && rt > 0 && rt <= kSplitTiles && R <= kSplitMaxRounds) {
-    np = max(1, min(min(G / rt, a.split_max), ksteps / kSplitMinStages));
-    // the last piece reads np partials: keep np at most sqrt(ksteps / 2),
-    // and two pieces only for long reductions
-    while (np > 1 && ksteps < 2 * np * np) --np;
-    if (np == 2 && ksteps < 64) np = 1;
-    np = U(np);
-  }
+  const int np = a.part != nullptr ? U(split_pieces(R, rt, G, ksteps, a.split_max)) : 1;
   const bool has_piece = np > 1 && slot < rt * np;
   const int nfull = U(np > 1 ? R : (slot < ntiles ? (ntiles - slot + G - 1) / G : 0));
   const int nmy = nfull + (has_piece ? 1 : 0);
@@ -879,7 +871,7 @@ hipError_t launch_fwd(FwdArgs a, hipStream_t stream) {
 
 // Pieces per split leftover tile at most (TTAMD_GEMM_SPLIT=1 turns the
 // split off, for A/B timing).
-static int split_max() {
+int split_max() {
   static const int v = [] {
     const char* e = getenv("TTAMD_GEMM_SPLIT");
     const int n = e ? atoi(e) : kSplitMaxPieces;

@@ -82,6 +82,8 @@ size_t gemm_workspace_bytes(int64_t M, int E);
 size_t gemm_plan_bytes(int64_t M, int E);
 // Largest token tile of the bf16 forward / dgrad GEMMs (tile plans are built for it).
 int gemm_fwd_tile_rows();
+void gemm_tiles(const int* counts, int E, int64_t weight_rows, int k, bool fp8, int* tile_rows, int* tile_cols,
+                int* pieces);
 // The next forward grouped-GEMM launch records these events around its main
 // kernel on its stream, then the probe disarms (nullptr, nullptr: disarm).
 void gemm_probe_arm(hipEvent_t start, hipEvent_t end);

@@ -610,6 +610,17 @@ def _gemm_ws(M: int, E: int, dev: torch.device) -> torch.Tensor:
     return _ws(_lib.load().ttamd_gemm_workspace_bytes(M, E), dev)
 
 
+def gemm_tiles(counts, weight_rows: int, k: int, fp8: bool = False) -> tuple[int, int, int]:
+    """(token rows, weight rows, tail pieces) of the tiles that a forward
+    grouped GEMM with these rows per expert runs on (ttamd_gemm_tiles; for
+    reports and tests, nothing is launched)."""
+    c = [int(v) for v in counts]
+    out = [ctypes.c_int() for _ in range(3)]
+    _lib.call("ttamd_gemm_tiles", (ctypes.c_int * len(c))(*c), len(c), weight_rows, k, int(fp8),
+              *[ctypes.byref(v) for v in out])
+    return tuple(v.value for v in out)
+
+
 def probe_next_gemm(start: "torch.cuda.Event | None", end: "torch.cuda.Event | None") -> None:
     """Arm the kernel timing probe (ttamd_probe_next_gemm): the next forward
     grouped-GEMM op (grouped_mm*, bf16 or fp8) records `start` and `end` on its
