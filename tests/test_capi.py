@@ -217,3 +217,28 @@ def test_gemm_tile_choice(counts, weight_rows, k, large):
     the rule, small_tile_cols)."""
     rows, cols, _ = _tiles(counts, weight_rows, k)
     assert (rows == 320) == large, (rows, cols)
+
+
+def _zipf(rows, experts, s=1.2):
+    w = [r ** -s for r in range(1, experts + 1)]
+    c = [int(rows * v / sum(w)) for v in w]
+    c[0] += rows - sum(c)
+    return c
+
+
+@pytest.mark.parametrize("counts,weight_rows,k,tile_rows", [
+    # DeepSeek-V3 shard w13 and w2, 72 and 56 rows per expert on average: an
+    # even load stays on the small tiles, a skewed one whose small tiles just
+    # pass a round goes to the large ones, one that passes it in both does not
+    ((72,) * 32, 4096, 7168, 128), (_zipf(2300, 28) + [0] * 4, 4096, 7168, 256), (_zipf(3199, 28) + [0] * 4, 4096, 7168, 128),
+    (_zipf(1800, 23) + [0] * 9, 7168, 2048, 256), ((56,) * 32, 7168, 2048, 128), ([800] * 4 + [0] * 28, 4096, 7168, 256),
+    # few experts: the fp8 stage times, not bf16's
+    ((500,) * 4, 2048, 4096, 128), ((1250,) * 4, 2048, 4096, 256), ((2000,) * 4, 2048, 4096, 256),
+    ((1000,), 4096, 7168, 128), ((3000,), 4096, 7168, 256),
+    # few rows and prefill
+    ((7,) * 28 + (0,) * 4, 4096, 7168, 64), ((200,), 7168, 2048, 64), ((1024,) * 32, 4096, 7168, 256),
+])
+def test_fp8_tile_choice(counts, weight_rows, k, tile_rows):
+    """Each load on the fp8 tiles that were measured ahead on it (times beside
+    fp8_pick_small and fp8_choice)."""
+    assert _tiles(counts, weight_rows, k, True)[0] == tile_rows

@@ -163,6 +163,28 @@ def _check_fp8(ops, counts, n, K, seed):
         assert_close(to_np(a), O.swiglu(h_ref, limit), 2 * TOL, "a")
 
 
+# rows per expert, N (or H), K of calls whose tile counts decide between the
+# 128-row and the 256-row tiles on the device, with the tile expected of the
+# store / scatter (N) and the SwiGLU (2 H) GEMM: both sides and both widths of
+# the small one, the same row total even and on few experts
+FP8_PICK_CASES = [
+    ((107,) * 24, 1920, 512, (128, 256), (128, 256)),
+    ((130,) * 10 + (90,) * 14, 1920, 384, (256, 256), (128, 256)),  # the same rows near enough: one more small round
+    ((97,) * 14, 1152, 384, (128, 128), (128, 256)),
+    ((120,) * 60, 640, 256, (128, 256), (128, 128)),
+    ((900,) * 8, 2048, 512, (256, 256), (256, 256)),
+    ((7000, 1, 129, 0, 33, 0, 0, 255), 1088, 256, (128, 128), (256, 256)),  # up rows straddle scale blocks
+]
+
+
+@pytest.mark.parametrize("i", range(len(FP8_PICK_CASES)))
+def test_fp8_tiles_chosen_by_the_plan(ops, i):
+    counts, n, K, tiles_n, tiles_h = FP8_PICK_CASES[i]
+    assert ops.gemm_tiles(counts, -(-n // 128) * 128, K, True)[:2] == tiles_n
+    assert ops.gemm_tiles(counts, 2 * (-(-n // 64) * 64), K, True)[:2] == tiles_h
+    _check_fp8(ops, counts, n, K, 400 + i)
+
+
 @pytest.mark.parametrize("R", [1, 4, 5, 8191, 8193])
 def test_fp8_row_quantiser_row_groups(ops, R):
     """Few rows run one per wave, many four per wave: the same codes and

@@ -160,23 +160,41 @@ static int small_tile_cols(int M, int E, int64_t cols, int k) {
   return 100 * (600 + std::max(small_time, stream)) > 107 * (600 + std::max(large_time, stream * 105 / 100)) ? 0 : small;
 }
 
-static int fp8_small_cols(int M, int E, int64_t cols, int64_t row_bytes) {
-  const int rows = small_tile_rows(M, E);
-  if (rows == 0) return 0;
+// The fp8 tiling: 64-row small tiles (rows 64) or large ones (256) where the
+// rows alone decide it, else 128-row small tiles or large ones by the plan's
+// tile counts (rows 128: fp8_pick_small, on the device).  Times as in
+// small_tile_cols, of the fp8 kernels: 0.01 us per stage of 128 k and tile of
+// full height 64 x 128 50, 64 x 256 83, 128 x 128 77, 128 x 256 110, 256 x 256
+// 164 and at least 97; with weights that stream from HBM, where a stage waits
+// for its rows, 60, 100, 100, 160 and at least 163 (32 experts of 4096 x 7168,
+// full rounds; the wider small tile then).  From 1 and 4 experts of 7168 x 2048, 4096 x 7168, 2048 x 1024
+// and 2048 x 4096 with 8 to 8000 rows.  Small against large, us: 4 experts of
+// 2048 x 4096, 2000 rows 49 against 67, 5000 rows 89 against 69, 8000 rows 95
+// against 67; one of 4096 x 7168, 1000 rows 57 against 110, 3000 rows 148
+// against 111.
+struct Fp8Choice {
+  int rows, cols, small_time;
+  bool stream;
+};
+static Fp8Choice fp8_choice(int M, int E, int64_t cols, int k) {
+  const int rows = small_tile_rows(M, E), stages = k / 128;
+  const bool stream = std::min(E, M) * cols * k > kSmallWeightBytes;
+  if (rows == 0) return {kFp8TileRows, 256, 0, stream};
   const int64_t G = (num_cus() + 7) & ~7;
-  auto qtiles = [&](int h) {
-    const int64_t hit = std::min(E, M);
-    return std::max<int64_t>(hit, (M + h - 1) / h + (hit - 1) / 3);
-  };
-  auto tiles = [&](int h, int c) { return qtiles(h) * ((cols + c - 1) / c); };
-  auto cost = [&](int h, int c, int64_t stage) { return (tiles(h, c) + G - 1) / G * stage; };
-  const int64_t c128 = cost(rows, 128, rows == 64 ? 50 : 66), c256 = cost(rows, 256, rows == 64 ? 85 : 108);
-  const int small = c128 < c256 ? 128 : 256;
-  if (M <= kSmallAvgRows * (int64_t)E) return small;
-  return std::min(E, M) * cols * row_bytes <= kSmallWeightBytes && tiles(kFp8TileRows, 256) < 2 * G &&
-                 std::min(c128, c256) < cost(kFp8TileRows, 256, 200)
-             ? small
-             : 0;
+  auto rounds = [&](int c) { return ceil_div(expected_qtiles(M, E, rows) * ceil_div(cols, c), G); };
+  if (rows == 64) {
+    const int64_t c128 = rounds(128) * (450 + (stream ? 60 : 50) * stages);
+    const int64_t c256 = rounds(256) * (493 + (stream ? 100 : 83) * stages);
+    const int64_t large_q = expected_qtiles(M, E, kFp8TileRows), large_tiles = large_q * ceil_div(cols, 256);
+    const int64_t large = ceil_div(large_tiles, G) * fp8_large_round(stages, stream, (int)ceil_div(M, large_q));
+    if (large_tiles < G && 100 * std::min(c128, c256) > 107 * large) return {kFp8TileRows, 256, 0, stream};
+    return {64, c128 < c256 ? 128 : 256, 0, stream};
+  }
+  const int t128 = 50 + 65 * stages, t256 = 100 + (stream ? 137 : 86) * stages;
+  const int h = (int)ceil_div(M, expected_qtiles(M, E, 128));
+  const bool narrow = !stream && rounds(128) * (t128 + fp8_small_rows(stages, 128, h)) <
+                                     rounds(256) * (t256 + fp8_small_rows(stages, 256, h));
+  return narrow ? Fp8Choice{128, 128, t128, false} : Fp8Choice{128, 256, t256, stream};
 }
 
 // The tiles a forward GEMM with these host counts runs on (ttamd_gemm_tiles).
@@ -184,16 +202,28 @@ void gemm_tiles(const int* counts, int E, int64_t weight_rows, int k, bool fp8, 
                 int* pieces) {
   int64_t M = 0;
   for (int e = 0; e < E; ++e) M += counts[e];
-  const int small = fp8 ? fp8_small_cols((int)M, E, weight_rows, k) : small_tile_cols((int)M, E, weight_rows, k);
-  *tile_rows = small ? small_tile_rows((int)M, E) : fp8 ? kFp8TileRows : kFwdTileRows;
-  *tile_cols = small ? small : 256;
   *pieces = 1;
-  if (small || fp8) return;
-  int64_t tiles = 0;
-  for (int e = 0; e < E; ++e) tiles += tiles_of(counts[e], kFwdTileRows);
-  tiles *= ceil_div(weight_rows, 256);
-  const int64_t G = (num_cus() + 7) & ~7;
-  if (tiles / G <= kSplitMaxRounds) *pieces = split_pieces((int)(tiles / G), (int)(tiles % G), (int)G, k / 64, split_max());
+  const int G = (num_cus() + 7) & ~7;
+  auto tiles_in = [&](int max_rows) {
+    int n = 0;
+    for (int e = 0; e < E; ++e) n += tiles_of(counts[e], max_rows);
+    return n;
+  };
+  if (fp8) {
+    const Fp8Choice c = fp8_choice((int)M, E, weight_rows, k);
+    const Fp8Pick p = {nullptr, nullptr, (int)ceil_div(weight_rows, c.cols), c.cols, c.small_time, (int)M, c.stream};
+    const bool small = c.rows == 64 || (c.rows == 128 && fp8_pick_small(p, tiles_in(128), tiles_in(kFp8TileRows),
+                                                                        (int)ceil_div(weight_rows, 256), k / 128, G));
+    *tile_rows = small ? c.rows : kFp8TileRows;
+    *tile_cols = small ? c.cols : 256;
+    return;
+  }
+  const int small = small_tile_cols((int)M, E, weight_rows, k);
+  *tile_rows = small ? small_tile_rows((int)M, E) : kFwdTileRows;
+  *tile_cols = small ? small : 256;
+  if (small) return;
+  const int64_t tiles = tiles_in(kFwdTileRows) * ceil_div(weight_rows, 256);
+  if (tiles / G <= kSplitMaxRounds) *pieces = split_pieces((int)(tiles / G), (int)(tiles % G), G, k / 64, split_max());
 }
 
 // plan: the tile plan; part: the partial-sum area of split leftover tiles
@@ -319,10 +349,11 @@ static hipError_t fp8(int epi, Fp8Args a, const int* offs, int E, int M, void* w
   hipError_t err = launch_tile_map(offs, E, M, kFp8TileRows, ws, true, stream);
   if (err != hipSuccess) return err;
   const TileTable tt = tile_table_in(ws, M, E);
-  const int small = fp8_small_cols(M, E, a.n_p, a.kred);
-  a.table = small ? tt.small_table : tt.table;
-  a.n_qtiles = small ? tt.small_count : tt.count;
-  return small ? launch_small_fp8_gemm(epi, a, tt.small_rows, small, stream) : launch_fp8_gemm(epi, a, stream);
+  const Fp8Choice c = fp8_choice(M, E, a.n_p, a.kred);
+  a.table = c.rows == 64 ? tt.small_table : tt.table;
+  a.n_qtiles = c.rows == 64 ? tt.small_count : tt.count;
+  const Fp8Pick p = {tt.small_table, tt.small_count, 0, c.cols, c.small_time, M, c.stream};
+  return launch_fp8_gemm(epi, a, p, c.rows, c.cols, stream);
 }
 
 static Fp8Args fp8_args(const void* xq, const float* sx, const void* wq, const float* sw, int M,

@@ -324,6 +324,47 @@ struct Fp8Args {
 // Token tiles of the fp8 GEMM have at most this many rows.
 constexpr int kFp8TileRows = 256;
 
+// Estimated time of one round of fp8 tiles of h token rows (0.01 us, k in
+// stages of 128): large tiles, and the small ones' share that grows with the
+// rows (on top of a time that depends on their form, fp8_choice in gemm.hip).
+// `stream`: the weights stream from HBM, and a stage waits for its rows.
+__host__ __device__ inline int fp8_large_round(int stages, bool stream, int h) {
+  const int waits = stream ? 60 + stages * 163 + h * (820 + 5 * stages) / 100 : 450 + 463 * h / 100 + stages * 97;
+  return std::max(waits, 300 + 463 * h / 100 + stages * 164 * h / 256);
+}
+__host__ __device__ inline int fp8_small_rows(int stages, int cols, int h) { return h * (385 + 9 * stages) * (cols / 128) / 100; }
+
+// Small (128-row) or large fp8 tiles by their rounds of G workgroups and the
+// time of a round of either.  The counts of tiles decide it, so it is made
+// where they are known, on the device: the rows per expert alone do not say
+// how a skewed load falls into rounds.  DeepSeek-V3 shard w13 (7168 -> 2 x
+// 2048, 16 weight tiles), us, small against large: 2300 rows over 32 experts
+// even 175 against 202 (2 rounds of both), Zipf(1.2) over 28 of them 247
+// against 196 (38 small token tiles, 3 rounds; 32 large, 2), 3199 rows
+// Zipf(1.2) over 28 248 against 280 (3 rounds of both), 3200 rows on 4 experts
+// 156 against 93.  Chosen by the average rows, the small side always ran.
+struct Fp8Pick {
+  const int4* small_table;
+  const int* small_count;
+  int small_np;    // weight-row tiles per small token tile
+  int small_cols;  // their weight rows
+  int small_time;  // one round of small tiles without fp8_small_rows
+  int rows;        // M
+  int stream;      // weights stream from HBM
+};
+__host__ __device__ inline bool fp8_pick_small(const Fp8Pick& p, int ns, int nl, int large_np, int stages, int G) {
+  // rounds of G tiles in units of 1 / 2G: after a full round, a last one of a
+  // share f takes (1 + f) / 2 of it (33 small tiles, 2.06 rounds, 221 us, 47,
+  // 2.94 rounds, 252; 32, 2 rounds, 171); within 7 % the small side stays
+  auto rounds = [&](int tiles) {
+    const int rest = tiles % G;
+    return (float)(tiles < G ? 2 * G : 2 * (tiles - rest) + (rest ? G + rest : 0));
+  };
+  const int small = p.small_time + fp8_small_rows(stages, p.small_cols, p.rows / std::max(ns, 1));
+  const int large = fp8_large_round(stages, p.stream != 0, p.rows / std::max(nl, 1));
+  return rounds(ns * p.small_np) * (float)(100 * small) <= rounds(nl * large_np) * (float)(107 * large);
+}
+
 int num_cus();
 
 // with_small: also the small-tile table, where small_tile_rows(M, E) > 0.
@@ -338,9 +379,9 @@ hipError_t launch_small_gemm(int epi, FwdArgs a, int tile_rows, int tile_cols, h
 int split_max();
 // dgrad GEMM (EPI_STORE or EPI_SWIGLU_BWD) over the same tile table.
 hipError_t launch_dgrad_gemm(int epi, const DgradGemm& g, hipStream_t stream);
-// fp8 forward GEMM over a tile table of at most kFp8TileRows rows per tile.
-hipError_t launch_fp8_gemm(int epi, const Fp8Args& a, hipStream_t stream);
-// Small-tile form (gemm_fp8_small.hip): tiles of at most `rows` token rows, `cols` weight rows.
-hipError_t launch_small_fp8_gemm(int epi, const Fp8Args& a, int rows, int cols, hipStream_t stream);
+// fp8 forward GEMM (gemm_fp8.hip).  rows 64: small tiles of 64 token rows x
+// `cols` weight rows, whose table is a.table; rows 128: small tiles of 128 x
+// `cols` (p) or the large ones (a), chosen on the device; 256: the large ones.
+hipError_t launch_fp8_gemm(int epi, const Fp8Args& a, const Fp8Pick& p, int rows, int cols, hipStream_t stream);
 
 }  // namespace ttamd

@@ -62,6 +62,7 @@
 #include "common.h"
 #include "dma_asm.h"
 #include "gemm_common.h"
+#include "gemm_fp8_small.h"
 #include "kernels.h"
 
 namespace ttamd {
@@ -107,8 +108,9 @@ constexpr int NPB16 = 4;
 constexpr int NJ16 = 8;
 constexpr int NBS = 2;
 
+// One workgroup's share of a GEMM over nqt token tiles of at most TQ rows.
 template <int EPI>
-__global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_kernel(const Fp8Args a) {
+__device__ __forceinline__ void run_large(const Fp8Args& a, int nqt) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wq = w >> 2;  // token half: rows 128 wq ..
@@ -117,7 +119,7 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_kernel(const Fp8Args a) {
   const int G = gridDim.x;
   const int b = blockIdx.x;
   const int slot = (b & 7) * (G >> 3) + (b >> 3);
-  const int ntiles = sload_int(a.n_qtiles) * a.np_tiles;
+  const int ntiles = nqt * a.np_tiles;
   const int nmy = slot < ntiles ? (ntiles - slot + G - 1) / G : 0;
   const int ksteps = a.kred / TKB;
   const int total = nmy * ksteps;
@@ -461,21 +463,76 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_kernel(const Fp8Args a) {
 }
 
 template <int EPI>
-hipError_t launch_fp8(const Fp8Args& a, hipStream_t stream) {
-  // set once per process (thread-safe static initialisation)
+__global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_kernel(const Fp8Args a) {
+  run_large<EPI>(a, sload_int(a.n_qtiles));
+}
+
+template <int EPI, int SQ, int STP>
+__global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_small_kernel(const Fp8Args a) {
+  fp8_small::run<EPI, SQ, STP>(a, a.table, sload_int(a.n_qtiles), a.np_tiles);
+}
+
+// The kernel's Fp8Args (its first argument) loaded where this is called: the
+// two sides of gg_fp8_pick_kernel would otherwise hold the union of their
+// arguments from the kernel's start, and spill scalars in their stage loops.
+__device__ __forceinline__ Fp8Args load_args() {
+  auto p = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  Fp8Args a;
+  __builtin_memcpy(&a, (const void*)p, sizeof(a));
+  return a;
+}
+
+// Both tilings, chosen by the tile counts of the plan: every workgroup sees
+// the same counts and takes the same side (fp8_pick_small says why).
+template <int EPI, int STP>
+__global__ __launch_bounds__(FTHREADS, 1) void gg_fp8_pick_kernel(const Fp8Args a, const Fp8Pick p) {
+  const int nl = sload_int(a.n_qtiles), ns = sload_int(p.small_count);
+  if (fp8_pick_small(p, ns, nl, a.np_tiles, a.kred / TKB, gridDim.x)) {
+    fp8_small::run<EPI, 128, STP>(load_args(), p.small_table, ns, p.small_np);
+  } else {
+    run_large<EPI>(load_args(), nl);
+  }
+}
+
+// LDS above the default limit, set once per process and kernel (thread-safe
+// static initialisation).
+template <auto KERNEL, typename... Args>
+hipError_t launch_lds(int lds, hipStream_t stream, const Args&... args) {
   static const hipError_t attr_err =
-      hipFuncSetAttribute((const void*)gg_fp8_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_TOTAL);
+      hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr_err != hipSuccess) return attr_err;
-  const int grid = (num_cus() + 7) & ~7;
-  return launch_k(true, gg_fp8_kernel<EPI>, dim3(grid), dim3(FTHREADS), LDS_TOTAL, stream, a);
+  return launch_k(true, KERNEL, dim3((num_cus() + 7) & ~7), dim3(FTHREADS), lds, stream, args...);
+}
+
+int small_np(int epi, const Fp8Args& a, int cols) {
+  return epi == EPI_SWIGLU ? ((int)a.hidden + cols / 2 - 1) / (cols / 2) : (a.n_p + cols - 1) / cols;
+}
+
+template <int EPI, int STP>
+hipError_t launch_small(Fp8Args a, hipStream_t stream) {
+  a.np_tiles = small_np(EPI, a, STP);
+  return launch_lds<gg_fp8_small_kernel<EPI, 64, STP>>(fp8_small::Geo<64, STP>::LDS, stream, a);
+}
+template <int EPI, int STP>
+hipError_t launch_pick(const Fp8Args& a, Fp8Pick p, hipStream_t stream) {
+  p.small_np = small_np(EPI, a, STP);
+  constexpr int lds = fp8_small::Geo<128, STP>::LDS > LDS_TOTAL ? fp8_small::Geo<128, STP>::LDS : LDS_TOTAL;
+  return launch_lds<gg_fp8_pick_kernel<EPI, STP>>(lds, stream, a, p);
+}
+template <int EPI>
+hipError_t launch_epi(const Fp8Args& a, const Fp8Pick& p, int rows, int cols, hipStream_t stream) {
+  if (rows == 64) return cols == 128 ? launch_small<EPI, 128>(a, stream) : launch_small<EPI, 256>(a, stream);
+  if (rows == 128) return cols == 128 ? launch_pick<EPI, 128>(a, p, stream) : launch_pick<EPI, 256>(a, p, stream);
+  return launch_lds<gg_fp8_kernel<EPI>>(LDS_TOTAL, stream, a);
 }
 
 }  // namespace
 
-hipError_t launch_fp8_gemm(int epi, const Fp8Args& a, hipStream_t stream) {
-  if (epi == EPI_SWIGLU) return launch_fp8<EPI_SWIGLU>(a, stream);
-  if (epi == EPI_SCATTER) return launch_fp8<EPI_SCATTER>(a, stream);
-  return launch_fp8<EPI_STORE>(a, stream);
+hipError_t launch_fp8_gemm(int epi, const Fp8Args& a, const Fp8Pick& p, int rows, int cols, hipStream_t stream) {
+  if (epi == EPI_SWIGLU) return launch_epi<EPI_SWIGLU>(a, p, rows, cols, stream);
+  if (epi == EPI_SCATTER) return launch_epi<EPI_SCATTER>(a, p, rows, cols, stream);
+  return launch_epi<EPI_STORE>(a, p, rows, cols, stream);
 }
 
 }  // namespace ttamd

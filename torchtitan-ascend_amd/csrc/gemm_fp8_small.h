@@ -26,13 +26,15 @@
 // -> 281, 1000 rows 385 -> 305, 3000 rows 430 -> 369; w13 at 200 rows 184 ->
 // 141 us (5.8 TB/s of weights; its tables and the two quantisations are the
 // rest).
+#pragma once
+
 #include "common.h"
 #include "dma_asm.h"
 #include "gemm_common.h"
 #include "kernels.h"
 
 namespace ttamd {
-namespace {
+namespace fp8_small {
 
 using namespace dma;
 
@@ -60,8 +62,9 @@ struct Geo {
   static_assert(LDS <= 160 * 1024, "LDS of a CU");
 };
 
+// One workgroup's share of a GEMM over nqt token tiles of at most TQ rows.
 template <int EPI, int TQ, int STP>
-__global__ __launch_bounds__(64 * SWAVES, 1) void gg_fp8_small_kernel(const Fp8Args a) {
+__device__ __forceinline__ void run(const Fp8Args& a, const int4* table, int nqt, int np_tiles) {
   using L = Geo<TQ, STP>;
   constexpr int NPB = L::NPB, NJ = L::NJ;
   constexpr int COLS = EPI == EPI_SWIGLU ? STP / 2 : STP;  // output columns per tile
@@ -73,8 +76,7 @@ __global__ __launch_bounds__(64 * SWAVES, 1) void gg_fp8_small_kernel(const Fp8A
   const int G = gridDim.x;
   const int b = blockIdx.x;
   auto U = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
-  const int nqt = sload_int(a.n_qtiles);
-  const int ntiles = nqt * a.np_tiles;
+  const int ntiles = nqt * np_tiles;
   const int ksteps = U(a.kred / SKB);
   // walk, tile order and k rotation as in gemm_small.hip
   const int R = U(ntiles / G);
@@ -85,8 +87,8 @@ __global__ __launch_bounds__(64 * SWAVES, 1) void gg_fp8_small_kernel(const Fp8A
   const int total = nmy * ksteps;
   auto tile_at = [&](int r, int& qt, int& pt) {
     const int t = r < R ? r * G + slot : R * G + b;
-    const int blk = t / (2 * a.np_tiles);
-    const int in_blk = t - blk * 2 * a.np_tiles;
+    const int blk = t / (2 * np_tiles);
+    const int in_blk = t - blk * 2 * np_tiles;
     const int gq = min(2, nqt - 2 * blk);
     pt = in_blk / gq;
     qt = 2 * blk + (in_blk - pt * gq);
@@ -106,7 +108,7 @@ __global__ __launch_bounds__(64 * SWAVES, 1) void gg_fp8_small_kernel(const Fp8A
   auto dma_tile = [&](int r) {
     int qt, pt;
     tile_at(r, qt, pt);
-    const int4 ti = sload_int4(a.table + qt);
+    const int4 ti = sload_int4(table + qt);
     const int qmax = ti.z - ti.y - 1;
     const int last = n_cols - 1 - pt * COLS;
 #pragma unroll
@@ -183,7 +185,7 @@ __global__ __launch_bounds__(64 * SWAVES, 1) void gg_fp8_small_kernel(const Fp8A
   for (int r = 0; r < nmy; ++r) {
     int qt, pt;
     tile_at(r, qt, pt);
-    const int4 ti = sload_int4(a.table + qt);
+    const int4 ti = sload_int4(table + qt);
     const int row0 = ti.y, row1 = ti.z;
     const int nblk = (row1 - row0 + 15) >> 4;  // 16-row token blocks of the tile
     floatx4_t acc[NPB][NJ];
@@ -284,31 +286,5 @@ __global__ __launch_bounds__(64 * SWAVES, 1) void gg_fp8_small_kernel(const Fp8A
   wait_vm<0>();  // DMAs past the end have landed before the workgroup exits
 }
 
-template <int EPI, int TQ, int STP>
-hipError_t launch_tile(Fp8Args a, hipStream_t stream) {
-  // set once per process (thread-safe static initialisation)
-  static const hipError_t attr_err = hipFuncSetAttribute((const void*)gg_fp8_small_kernel<EPI, TQ, STP>,
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, Geo<TQ, STP>::LDS);
-  if (attr_err != hipSuccess) return attr_err;
-  constexpr int COLS = EPI == EPI_SWIGLU ? STP / 2 : STP;
-  const int n = EPI == EPI_SWIGLU ? (int)a.hidden : a.n_p;
-  a.np_tiles = (n + COLS - 1) / COLS;
-  const int grid = (num_cus() + 7) & ~7;
-  return launch_k(true, gg_fp8_small_kernel<EPI, TQ, STP>, dim3(grid), dim3(64 * SWAVES), Geo<TQ, STP>::LDS, stream, a);
-}
-
-template <int EPI>
-hipError_t launch_epi(const Fp8Args& a, int rows, int cols, hipStream_t stream) {
-  if (rows == 64) return cols == 128 ? launch_tile<EPI, 64, 128>(a, stream) : launch_tile<EPI, 64, 256>(a, stream);
-  return cols == 128 ? launch_tile<EPI, 128, 128>(a, stream) : launch_tile<EPI, 128, 256>(a, stream);
-}
-
-}  // namespace
-
-hipError_t launch_small_fp8_gemm(int epi, const Fp8Args& a, int rows, int cols, hipStream_t stream) {
-  if (epi == EPI_SWIGLU) return launch_epi<EPI_SWIGLU>(a, rows, cols, stream);
-  if (epi == EPI_SCATTER) return launch_epi<EPI_SCATTER>(a, rows, cols, stream);
-  return launch_epi<EPI_STORE>(a, rows, cols, stream);
-}
-
+}  // namespace fp8_small
 }  // namespace ttamd
