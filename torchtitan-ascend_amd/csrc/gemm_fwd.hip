@@ -277,12 +277,20 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     }
     // Weight rows a multiple of 4 KB apart: tiles at the same k ask the same
     // HBM channels, so each expert starts its k walk elsewhere (the tiles of
-    // one expert keep sharing their lines).  128 rows per expert of 768 x
-    // 2048, where the weights' stream is the bound: w13 197 -> 161 us; 256
-    // rows 233 -> 223, 512 rows unchanged; offsets per weight tile as well
-    // lose the shared token lines (512 rows 382 -> 407).  A split tile's
-    // pieces keep their k ranges.
-    if constexpr (!PT) d_rot = (a.ldp * 2) % 4096 == 0 && r < nfull ? U(3 * ti.x % ksteps) : 0;
+    // one expert keep sharing their lines).  Against one k order for all, us:
+    // 128 experts of 1536 x 2048, 128 rows each 199 -> 160, 256 rows 228 ->
+    // 202, 512 rows 357 -> 353, 1024 rows unchanged; 32 of 7168 x 2048, 128
+    // rows 239 -> 200, 512 rows 424 -> 426; 32 of 4096 x 4096, 128 rows 250 ->
+    // 198; 16 of 4096 x 6144, 192 rows 203 -> 174.  Not for rows of 16 KB and
+    // more, where it loses with few rows per expert and gains nothing with
+    // many: 16 of 5120 x 8192, 128 rows 286 -> 299, 512 rows 589 -> 590; 8 of
+    // 8192 x 8192, 192 rows 218 -> 242.  Offsets per weight tile as well lose
+    // the shared token lines (512 rows 382 -> 407).  A split tile's pieces keep
+    // their k ranges.
+    if constexpr (!PT) {
+      const uint32_t row = (uint32_t)a.ldp * 2;
+      d_rot = row % 4096 == 0 && row < 16384 && r < nfull ? U(3 * ti.x % ksteps) : 0;
+    }
     d_r = r;
   };
   // A stage's DMA is issued in two parts: the weight rows (P) at the stage
