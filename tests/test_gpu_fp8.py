@@ -188,9 +188,12 @@ TILE_HEIGHTS = np.array([1, 16, 17, 31, 32, 33, 48, 64, 65, 96, 97, 127, 128, 12
 
 
 @pytest.mark.parametrize("epi", ["store", "swiglu", "scatter"])
-def test_fp8_every_tile_height(ops, epi):
+@pytest.mark.parametrize("times", [1, 3])  # once: the 128-row tiles; three times: past their range, the 256-row ones
+def test_fp8_every_tile_height(ops, epi, times):
     rng = np.random.default_rng(91)
-    counts = TILE_HEIGHTS
+    counts = np.tile(TILE_HEIGHTS, times)
+    for weight_rows in (256, 384):
+        assert ops.gemm_tiles(counts, weight_rows, 256, True)[0] == (128 if times == 1 else 256)
     E, M = counts.size, int(counts.sum())
     offs = _offs(counts)
     announce(f"fp8 tile heights epi={epi} M={M} E={E}")

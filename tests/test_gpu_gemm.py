@@ -95,12 +95,13 @@ def test_grouped_mm_swiglu(ops, M, E, D, H, kind, limit):
     assert_close(to_np(a), O.swiglu(to_np(h), limit), 1e-2, "to_np(a)")
 
 
-@pytest.mark.parametrize("counts,H", [((400, 100), 2304), ((400, 0, 100, 333), 2304), ((50,), 2304)])
+@pytest.mark.parametrize("counts,H", [((400, 100), 2304), ((400, 0, 100, 333), 2304), ((50,), 2304),
+                                      ((8200, 320), 2304), ((8300, 0, 100, 1), 2304)])
 def test_grouped_mm_swiglu_paired_walk_odd_tiles(ops, counts, H):
     """The SwiGLU kernels walk the token tiles in pairs (weight tile major
     inside a pair); with an odd token-tile count the last pair has one tile,
     and with H / 128 = 18 weight tiles a pair spans more than one XCD's 32
-    slots.  Every tile must still be computed exactly once: compared in
+    slots (small tiles up to 8192 rows here, the 320 x 256 ones above).  Every tile must still be computed exactly once: compared in
     full with the oracle, per row."""
     rng = np.random.default_rng(sum(counts) + H)
     counts = np.array(counts, np.int64)
@@ -108,6 +109,7 @@ def test_grouped_mm_swiglu_paired_walk_odd_tiles(ops, counts, H):
     x = rand_bf16(rng, (M, D))
     w13 = rand_bf16(rng, (E, 2 * H, D), 0.08)
     announce(f"swiglu paired walk counts={tuple(counts)} H={H}")
+    assert (ops.gemm_tiles(counts, 2 * H, D)[0] == 320) == (M > 8192)
     a, h = ops.grouped_mm_swiglu(bf16_dev(x), bf16_dev(w13), _offs(counts), None, save_h=True)
     h_ref = O.bf16_round(_gmm_ref(x, w13, counts))
     assert_close(to_np(h), h_ref, TOL, "h")

@@ -22,9 +22,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T,D,H,E,K,func,norm,before", [
     (2048, 256, 512, 8, 1, "sigmoid", False, True),
     (1024, 512, 256, 32, 8, "softmax", True, False),
-    # w13: 64 tiles of 32 k stages on 256 CUs, each split into 4 pieces, so
-    # the replays reuse the plan's arrival counters
-    (1024, 2048, 1024, 8, 2, "softmax", True, False),
+    # w13: 40 x 8 tiles of 32 k stages, 64 of them left over after a full round
+    # of 256 CUs and split into 4 pieces each, so the replays reuse the plan's
+    # arrival counters
+    (5200, 2048, 1024, 8, 2, "softmax", True, False),
 ])
 def test_graph_replays_equal_eager(ops, T, D, H, E, K, func, norm, before):
     G = importlib.import_module("torchtitan-ascend_amd.graph")
@@ -47,5 +48,9 @@ def test_graph_replays_equal_eager(ops, T, D, H, E, K, func, norm, before):
             torch.cuda.synchronize()
             want = eager(x)
             torch.cuda.synchronize()
+            if T == 5200:
+                counts = ops.router_route(x, wr, K, func, norm)[2].counts.tolist()
+                rows, _, pieces = ops.gemm_tiles(counts, 2 * H, D)
+                assert rows == 320 and pieces > 1, "the case's w13 does not split"
             assert torch.equal(got, want), f"replay {i} differs from the eager step"
             assert not torch.equal(other, want)

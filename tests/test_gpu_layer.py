@@ -201,9 +201,10 @@ def test_c4_deepseek_shard_full_size_sampled(pkg, ops):
 
 @pytest.mark.parametrize("T,D,H,gated,limit", [(300, 256, 128, True, None), (1000, 512, 192, False, None),
                                               (77, 128, 64, True, 0.4), (64, 128, 64, False, 0.0),
-                                              # w2: 7 x 8 tiles of 64 k stages, split into 4 pieces
-                                              # (the accumulating, gated epilogue runs once per tile)
-                                              (2048, 2048, 4096, True, None)])
+                                              (2048, 2048, 4096, True, None),
+                                              # w2: 10 tiles of 128 k stages, split into 8 pieces (the
+                                              # accumulating, gated epilogue runs once per tile)
+                                              (64, 2560, 8192, True, None)])
 def test_shared_expert_add_vs_oracle(pkg, ops, T, D, H, gated, limit):
     """Shared expert fused into the combine (the shared w2 GEMM adds into the
     routed output in its epilogue) against the oracle's block tail."""
@@ -214,6 +215,7 @@ def test_shared_expert_add_vs_oracle(pkg, ops, T, D, H, gated, limit):
     routed = rand_bf16(rng, (T, D))
     gl = (rng.standard_normal(T) * 2).astype(np.float32) if gated else None
     announce(f"shared_expert_add T={T} D={D} H={H} gated={gated} limit={limit}")
+    assert H != 8192 or ops.gemm_tiles((T,), D, H) == (320, 256, 8)
     out = bf16_dev(routed)
     ops.shared_expert_add(out, bf16_dev(x), bf16_dev(w13), bf16_dev(w2),
                           None if gl is None else torch.from_numpy(gl).to(DEV), limit)

@@ -342,6 +342,12 @@ def _bf16_ulp(v):
     (300, 512, 16, 1, "sigmoid", False, False),     # Llama4-Scout expert count
     (257, 384, 256, 8, "sigmoid", True, True),      # DeepSeek-V3 count, expert bias
     (33, 128, 60, 4, "softmax", False, False),      # ragged token tile, E not a block multiple
+    # few tokens: up to two token tiles take up to 16 slices of D
+    (2, 2048, 128, 8, "softmax", True, False),      # 16 slices
+    (32, 2112, 128, 8, "softmax", True, False),     # 11 slices of 3 stages
+    (130, 2048, 64, 4, "softmax", True, True),      # two token tiles, the second ragged
+    (256, 1280, 60, 4, "sigmoid", False, False),    # 10 slices, E not a block multiple
+    (1, 7168, 256, 8, "sigmoid", True, True),       # 16 slices of 7 stages
 ])
 def test_router_fused_vs_oracle(ops, T, D, E, K, func, norm, bias):
     """Fused gate GEMM + top-k: the bf16 logits match the oracle's F.linear to

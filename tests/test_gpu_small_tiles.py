@@ -1,9 +1,14 @@
-"""GPU parity of the small-tile grouped GEMM (few rows per expert, few tiles).
+"""GPU parity of the grouped GEMMs on each of their tilings.
 
-Cases sit at the edges of its choices: 64- and 128-row tiles, 128 and 256
-weight rows (the last tile half full), one row, a full tile and one row
-more, empty experts, k of one stage and of fewer stages than the ring, and
-rows a multiple of 4 KB apart (the k walk then starts elsewhere per tile).
+The small tiles (few rows per expert, few tiles): cases at the edges of their
+choices, 64- and 128-row tiles, 128 and 256 weight rows (the last tile half
+full), one row, a full tile and one row more, empty experts, k of one stage
+and of fewer stages than the ring, and rows a multiple of 4 KB apart (the k
+walk then starts elsewhere per tile).  The large ones (320 x 256, in fp8 256
+x 256): every token-block count, weight rows that leave the last tile part
+full, few k stages, the clamp and the saved pre-activation.  Each case names
+the tile it is meant for, asserted from the library's own choice.
+
 Tolerance: the inputs are bf16 and the sums fp32, so an output is off by
 its bf16 rounding (2^-9 relative, and the pre-activation's once more through
 the SwiGLU); 1e-2 of the row's largest value covers both.
@@ -20,34 +25,53 @@ from oracle import moe_oracle as O
 pytestmark = pytest.mark.gpu
 TOL = 1e-2
 
-# rows per expert, N (or H for the SwiGLU: 2 H weight rows), K
+# rows per expert, N (or H for the SwiGLU: 2 H weight rows), K, and the tile
+# of the store / scatter (N) and of the SwiGLU (2 H) GEMM
 CASES = [
-    ((1,), 128, 64),                                 # one row, one k stage
-    ((0, 1, 0, 2, 1), 192, 2048),                    # 64 x 128 tiles, rotated k walk
-    ((64, 65, 33, 1, 0, 63), 320, 192),              # 64-row tiles and one row past
-    ((5,) * 300, 384, 320),                          # more than one round, fewer stages than the ring
-    ((9,) * 200 + (0,) * 20 + (64,) * 3, 1152, 256),   # 64 x 256 tiles, half-full last tile
-    ((128, 129, 97, 1, 300, 0, 31), 448, 384),       # 128 x 128 tiles, one row past
-    ((90, 100, 128, 70, 96) * 26, 1152, 2048),         # 128 x 256 tiles, whole and partial rounds, rotated
-    ((700, 1300), 640, 1024),                        # more rows per expert, tiles too few for the large kernel
+    ((1,), 128, 64, (64, 128), (64, 128)),                        # one row, one k stage
+    ((0, 1, 0, 2, 1), 192, 2048, (64, 128), (64, 128)),           # rotated k walk
+    ((64, 65, 33, 1, 0, 63), 320, 192, (64, 128), (64, 128)),     # 64-row tiles and one row past
+    ((5,) * 300, 384, 320, (64, 128), (64, 256)),                 # more than one round, fewer stages than the ring
+    ((9,) * 200 + (0,) * 20 + (64,) * 3, 1664, 256, (64, 256), (64, 256)),  # last 256-row tile of N half full
+    ((9,) * 200 + (0,) * 20 + (64,) * 3, 448, 256, (64, 256), (64, 256)),   # ... and of H (H % 128 == 64)
+    ((128, 129, 97, 1, 300, 0, 31, 128, 90), 448, 384, (128, 128), (128, 128)),  # 128-row tiles and one row past
+    ((90, 100, 128, 70, 96) * 26, 1152, 2048, (128, 256), (128, 256)),  # whole and partial rounds, rotated, N half full
+    ((128, 129, 97, 1, 300, 0, 31) * 2, 1216, 256, (128, 128), (128, 256)),  # H % 128 == 64
+    ((700, 1300), 640, 1024, (128, 128), (128, 128)),             # more rows per expert, too few tiles for the large kernel
+]
+
+# every 32-row token block count, one row past a tile, tall experts in several
+# tiles of near-equal height, empty ones; twice, so that the row count is past
+# the small tiles' range
+HEIGHTS = (1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 256, 257, 288, 289, 319, 320, 321, 0, 640, 700) * 2
+LARGE = (320, 256)
+LARGE_CASES = [
+    (HEIGHTS, 192, 64, LARGE, LARGE),                             # one k stage; H % 128 == 64
+    (HEIGHTS[::-1], 320, 128, LARGE, LARGE),                      # two stages; last tile of H and of N half full
+    (HEIGHTS, 640, 192, LARGE, LARGE),                            # three stages; N half full
+    ((8200, 0, 100), 448, 2048, LARGE, LARGE),                    # 26 tiles of one expert, rotated k walk
 ]
 
 
+ALL_CASES = CASES + LARGE_CASES
+
+
 def _case(i):
-    counts, n, k = CASES[i]
+    counts, n, k, tile_n, tile_2h = ALL_CASES[i]
     counts = np.array(counts, np.int64)
     rng = np.random.default_rng(100 + i)
-    return counts, int(counts.sum()), len(counts), n, k, rng
+    return counts, int(counts.sum()), len(counts), n, k, rng, tile_n, tile_2h
 
 
 def _offs(counts):
     return torch.from_numpy(np.cumsum(counts).astype(np.int32)).to(DEV)
 
 
-@pytest.mark.parametrize("i", range(len(CASES)))
+@pytest.mark.parametrize("i", range(len(ALL_CASES)))
 @pytest.mark.parametrize("limit", [None, 0.5])
 def test_small_swiglu(ops, i, limit):
-    counts, M, E, H, D, rng = _case(i)
+    counts, M, E, H, D, rng, _, tile = _case(i)
+    assert ops.gemm_tiles(counts, 2 * H, D)[:2] == tile
     T = (M + 1) // 2
     tok, w13 = rand_bf16(rng, (T, D)), rand_bf16(rng, (E, 2 * H, D), 0.05)
     src = rng.integers(0, 2 * T, M).astype(np.int32)
@@ -63,10 +87,11 @@ def test_small_swiglu(ops, i, limit):
         assert torch.equal(a, a2) and torch.equal(h, h2), "gathered rows differ from the same rows given in order"
 
 
-@pytest.mark.parametrize("i", range(len(CASES)))
+@pytest.mark.parametrize("i", range(len(ALL_CASES)))
 def test_small_store_and_scatter(ops, i):
-    counts, M, E, N, K, rng = _case(i)
+    counts, M, E, N, K, rng, tile, _ = _case(i)
     N = -(-N // 128) * 128
+    assert ops.gemm_tiles(counts, N, K)[:2] == tile
     x, w = rand_bf16(rng, (M, K)), rand_bf16(rng, (E, N, K), 0.05)
     dest = rng.permutation(M).astype(np.int32)
     scale = rng.random(M).astype(np.float32)
@@ -80,9 +105,11 @@ def test_small_store_and_scatter(ops, i):
     assert_close(to_np(out), ref, TOL, "scatter")
 
 
-@pytest.mark.parametrize("T,D,H", [(1, 128, 64), (70, 256, 192), (900, 512, 448)])
-def test_small_shared_expert(ops, T, D, H):
+@pytest.mark.parametrize("T,D,H,tile_rows", [(1, 128, 64, 64), (70, 256, 192, 64), (900, 512, 448, 128),
+                                             (8300, 384, 192, 320)])
+def test_small_shared_expert(ops, T, D, H, tile_rows):
     """The accumulating, gated epilogue (one expert with every row)."""
+    assert ops.gemm_tiles((T,), D, H)[0] == tile_rows
     rng = np.random.default_rng(T)
     x, w13, w2 = rand_bf16(rng, (T, D)), rand_bf16(rng, (1, 2 * H, D), 0.05), rand_bf16(rng, (1, D, H), 0.05)
     base, gate = rand_bf16(rng, (T, D)), rng.standard_normal(T).astype(np.float32)
@@ -93,24 +120,27 @@ def test_small_shared_expert(ops, T, D, H):
     assert_close(to_np(out), base + y, TOL, "out")
 
 
-# rows per expert, N (or H), K (a multiple of 128) of the fp8 form
+# The same of the fp8 form: K a multiple of 128
 FP8_CASES = [
-    ((1,), 128, 128),                                 # one row, one k stage
-    ((0, 1, 0, 2, 1), 192, 4096),                    # 64 x 128 tiles, up rows straddle scale blocks, rotated k walk
-    ((64, 65, 33, 1, 0, 17, 16, 63), 320, 384),      # 64-row tiles and one row past, 16-row block edges
-    ((9,) * 200 + (0,) * 20 + (64,) * 3, 1152, 256),   # 64 x 256 tiles, half-full last tile
-    ((128, 129, 97, 1, 300, 0, 31), 448, 640),       # 128 x 128 tiles, one row past
-    ((90, 100, 128, 70, 96) * 26, 1152, 512),          # 128 x 256 tiles, whole and partial rounds
+    ((1,), 128, 128, (64, 128), (64, 128)),                       # one row, one k stage
+    ((0, 1, 0, 2, 1), 192, 4096, (64, 128), (64, 128)),           # up rows straddle scale blocks, rotated k walk
+    ((64, 65, 33, 1, 0, 17, 16, 63), 320, 384, (64, 128), (64, 128)),  # 64-row tiles and one row past, 16-row block edges
+    ((9,) * 200 + (0,) * 20 + (64,) * 3, 1152, 256, (64, 256), (64, 256)),  # last 256-row tile of N half full
+    ((9,) * 200 + (0,) * 20 + (64,) * 3, 448, 256, (64, 256), (64, 256)),   # ... and of H (H % 128 == 64)
+    ((128, 129, 97, 1, 300, 0, 31, 128, 90), 448, 640, (128, 128), (128, 128)),  # 128-row tiles and one row past
+    ((90, 100, 128, 70, 96) * 26, 1152, 512, (128, 128), (128, 256)),  # whole and partial rounds
 ]
 
 
 # The same of the 256 x 256 fp8 tiles: every 16-row block count in both halves,
 # walks of 1 to 4 tiles per workgroup, with 1 to 3 k stages of 128
 FP8_HEIGHTS = (1, 16, 17, 40, 64, 97, 128, 129, 144, 161, 200, 230, 256, 257, 300, 512)
+FP8_LARGE = (256, 256)
 FP8_LARGE_CASES = [
-    (FP8_HEIGHTS * 4, 3072, 128),
-    (FP8_HEIGHTS * 4, 1152, 256),
-    (FP8_HEIGHTS[::-1] * 4, 1024, 384),
+    (FP8_HEIGHTS * 4, 3072, 128, FP8_LARGE, FP8_LARGE),
+    (FP8_HEIGHTS * 4, 1152, 256, FP8_LARGE, FP8_LARGE),
+    (FP8_HEIGHTS[::-1] * 4, 1024, 384, FP8_LARGE, FP8_LARGE),
+    (FP8_HEIGHTS * 4, 320, 256, FP8_LARGE, FP8_LARGE),            # H % 128 == 64: up rows straddle scale blocks
 ]
 
 
@@ -129,12 +159,13 @@ def test_large_fp8_stage_pipeline(ops, i):
     _check_fp8(ops, *FP8_LARGE_CASES[i], 300 + i)
 
 
-def _check_fp8(ops, counts, n, K, seed):
+def _check_fp8(ops, counts, n, K, tile_n, tile_2h, seed):
     counts = np.array(counts, np.int64)
     M, E = int(counts.sum()), len(counts)
     offs_h, od = np.cumsum(counts), _offs(counts)
     rng = np.random.default_rng(seed)
     H, N = -(-n // 64) * 64, -(-n // 128) * 128
+    assert (ops.gemm_tiles(counts, N, K, True)[:2], ops.gemm_tiles(counts, 2 * H, K, True)[:2]) == (tile_n, tile_2h)
     x = bf16_dev(rand_bf16(rng, (M, K)))
     announce(f"fp8 tiles M={M} E={E} n={n} K={K}")
     xq, sx = ops.quantize_fp8_rows(x)
@@ -179,10 +210,7 @@ FP8_PICK_CASES = [
 
 @pytest.mark.parametrize("i", range(len(FP8_PICK_CASES)))
 def test_fp8_tiles_chosen_by_the_plan(ops, i):
-    counts, n, K, tiles_n, tiles_h = FP8_PICK_CASES[i]
-    assert ops.gemm_tiles(counts, -(-n // 128) * 128, K, True)[:2] == tiles_n
-    assert ops.gemm_tiles(counts, 2 * (-(-n // 64) * 64), K, True)[:2] == tiles_h
-    _check_fp8(ops, counts, n, K, 400 + i)
+    _check_fp8(ops, *FP8_PICK_CASES[i], 400 + i)
 
 
 @pytest.mark.parametrize("R", [1, 4, 5, 8191, 8193])

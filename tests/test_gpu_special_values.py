@@ -43,10 +43,12 @@ def _offs(counts):
 
 
 @pytest.mark.parametrize("limit", [None, 0.5])
-def test_swiglu_forward_nan_and_inf_rows(ops, limit):
+@pytest.mark.parametrize("counts,tile_rows", [((150, 0, 200, 90), 64), ((150, 0, 200, 90, 8000), 320)])
+def test_swiglu_forward_nan_and_inf_rows(ops, counts, tile_rows, limit):
     rng = np.random.default_rng(4100)
-    counts = np.array([150, 0, 200, 90], np.int64)
+    counts = np.array(counts, np.int64)
     M, E, D, H = int(counts.sum()), len(counts), 256, 192
+    assert ops.gemm_tiles(counts, 2 * H, D)[0] == tile_rows
     x = rand_bf16(rng, (M, D))
     x[5, :] = np.nan          # h row all NaN
     x[160, 7] = np.inf        # h row +-inf by the sign of w13[e][:, 7]
@@ -64,13 +66,15 @@ def test_swiglu_forward_nan_and_inf_rows(ops, limit):
 
 
 @pytest.mark.parametrize("limit", [None, 0.5])
-def test_fp8_swiglu_forward_nan_row(ops, limit):
+@pytest.mark.parametrize("counts,tile_rows", [((300, 212), 64), ((300, 212, 600), 128), ((300, 212, 7900), 256)])
+def test_fp8_swiglu_forward_nan_row(ops, counts, tile_rows, limit):
     """A NaN activation scale (one k block of one token row) makes that
     row's h NaN in the oracle's dequantise-then-GEMM; the kernel applies the
     scale to the block's partial sum, which gives the same NaN."""
     rng = np.random.default_rng(4200)
-    counts = np.array([300, 212], np.int64)
+    counts = np.array(counts, np.int64)
     M, E, D, H = int(counts.sum()), len(counts), 512, 256
+    assert ops.gemm_tiles(counts, 2 * H, D, True)[0] == tile_rows
     x = rand_bf16(rng, (M, D))
     w = rand_bf16(rng, (E, 2 * H, D), 0.02)
     xq, sx = O.quantize_fp8_rows(x)

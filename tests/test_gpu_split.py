@@ -4,8 +4,9 @@ The persistent walk runs R full rounds of one tile per workgroup; the rt
 tiles left over are cut along k into np pieces that run on the idle
 workgroups, and the last piece of a tile to arrive adds every piece's fp32
 partial sums in piece order before the epilogue.  Each case below is sized
-so that its leftover tiles are split on the device at hand (asserted from
-the device's CU count), and is checked against the oracle per row, for
+so that its leftover tiles are split on the device at hand (asserted: the
+forward ones by ops.gemm_tiles, which also says that the call runs on the 320
+x 256 tiles and not on the small ones, which have no split), and is checked against the oracle per row, for
 bit-identical results over repeated calls (the sum order does not depend
 on which piece arrives last), and, through the C-ABI, for the plan's
 arrival counters being back at zero afterwards.  Tolerance as the other
@@ -53,10 +54,13 @@ def _offs(counts):
     return torch.from_numpy(np.cumsum(counts).astype(np.int32)).to(DEV)
 
 
-def _expect_split(counts, n_wtiles: int, kred: int) -> None:
+def _expect_split(counts, n_wtiles: int, kred: int, ops=None) -> None:
+    """ops: a forward GEMM (the dgrad ones always run on the 320 x 256 tiles)."""
     ntiles = _qtiles(counts) * n_wtiles
     n = _pieces(ntiles, kred // 64)
     assert n > 1, f"case does not split on this device ({ntiles} tiles, {kred // 64} k stages, grid {_grid()})"
+    if ops is not None:
+        assert ops.gemm_tiles(counts, n_wtiles * 256, kred) == (320, 256, n)
 
 
 def _repeat_identical(fn, n=2):
@@ -69,15 +73,20 @@ def _repeat_identical(fn, n=2):
 
 
 # counts: every expert's rows fit one tile except where stated
-COUNTS = (320, 320, 200)
+COUNTS = (320, 320, 200)  # dgrad
+# forward: tiles of 9, 2 and 4 token blocks and an expert without rows; with
+# 128 stages 24 tiles in 8 pieces
+FWD_COUNTS = (260, 33, 0, 97)
+# one full round and 40 leftover tiles of 4, 9 and 10 token blocks
+FWD_ROUND = (320,) * 24 + (257,) * 5 + (97,) * 8
 
 
-@pytest.mark.parametrize("counts,N,K", [(COUNTS, 2048, 4096),          # 24 tiles, 64 stages: 5 pieces
+@pytest.mark.parametrize("counts,N,K", [(FWD_COUNTS, 2048, 8192),
                                         ((320,) * 35, 2048, 1600)])   # 280 tiles: one full round + 24, 3 pieces
 def test_split_grouped_mm(ops, counts, N, K):
     counts = np.array(counts, np.int64)
     M, E = int(counts.sum()), len(counts)
-    _expect_split(counts, N // 256, K)
+    _expect_split(counts, N // 256, K, ops)
     rng = np.random.default_rng(M + N + K)
     x, w = rand_bf16(rng, (M, K)), rand_bf16(rng, (E, N, K), 0.05)
     announce(f"split grouped_mm M={M} E={E} N={N} K={K}")
@@ -87,9 +96,9 @@ def test_split_grouped_mm(ops, counts, N, K):
 
 
 def test_split_counters_back_at_zero(ops):
-    counts = np.array(COUNTS, np.int64)
-    M, E, N, K = int(counts.sum()), len(counts), 2048, 4096
-    _expect_split(counts, N // 256, K)
+    counts = np.array(FWD_COUNTS, np.int64)
+    M, E, N, K = int(counts.sum()), len(counts), 2048, 8192
+    _expect_split(counts, N // 256, K, ops)
     rng = np.random.default_rng(5)
     x, w = bf16_dev(rand_bf16(rng, (M, K))), bf16_dev(rand_bf16(rng, (E, N, K), 0.05))
     lib = ops._lib.load()
@@ -108,11 +117,11 @@ def test_split_counters_back_at_zero(ops):
     assert_close(to_np(out), ref, TOL, "out")
 
 
-@pytest.mark.parametrize("limit", [None, 0.75])
-def test_split_swiglu(ops, limit):
-    counts = np.array(COUNTS, np.int64)
-    M, E, D, H = int(counts.sum()), len(counts), 4096, 1024
-    _expect_split(counts, H // 128, D)
+@pytest.mark.parametrize("counts,D,limit", [(FWD_COUNTS, 8192, None), (FWD_COUNTS, 8192, 0.75), (FWD_ROUND, 2048, 0.75)])
+def test_split_swiglu(ops, counts, D, limit):
+    counts = np.array(counts, np.int64)
+    M, E, H = int(counts.sum()), len(counts), 1024
+    _expect_split(counts, H // 128, D, ops)
     rng = np.random.default_rng(11)
     x, w13 = rand_bf16(rng, (M, D)), rand_bf16(rng, (E, 2 * H, D), 0.05)
     announce(f"split swiglu limit={limit}")
@@ -124,11 +133,11 @@ def test_split_swiglu(ops, limit):
 
 
 def test_split_swiglu_gather(ops):
-    counts = np.array(COUNTS, np.int64)
+    counts = np.array(FWD_COUNTS, np.int64)
     K = 2
-    M, E, D, H = int(counts.sum()), len(counts), 2048, 1024
+    M, E, D, H = int(counts.sum()), len(counts), 8192, 1024
     T = M // K
-    _expect_split(counts, H // 128, D)
+    _expect_split(counts, H // 128, D, ops)
     rng = np.random.default_rng(12)
     labels = rng.permutation(np.repeat(np.arange(E), counts))
     sidx = O.stable_order(labels, E).astype(np.int32)
@@ -142,9 +151,9 @@ def test_split_swiglu_gather(ops):
 
 
 def test_split_unpermute_scatter(ops):
-    counts = np.array(COUNTS, np.int64)
-    M, E, D, H = int(counts.sum()), len(counts), 2048, 2048
-    _expect_split(counts, D // 256, H)
+    counts = np.array(FWD_COUNTS, np.int64)
+    M, E, D, H = int(counts.sum()), len(counts), 2048, 8192
+    _expect_split(counts, D // 256, H, ops)
     rng = np.random.default_rng(13)
     a, w2 = rand_bf16(rng, (M, H)), rand_bf16(rng, (E, D, H), 0.05)
     dest = rng.permutation(M).astype(np.int32)
