@@ -58,9 +58,10 @@ inline int max_row_tiles(int M, int E) { return M / kTileRows + E + 1; }
 // rows at most, 128 or 256 weight rows.  Whether a GEMM of a plan takes it,
 // and with how many weight rows, is small_tile_cols' choice (gemm.hip); the
 // table exists wherever it could be chosen.  64-row tiles for experts that
-// mostly fit one, and for few rows in all (one expert of 7168 x 2048, 200
-// rows: 71 us against 94 with 128-row tiles; from ~1000 rows the 128-row
-// tiles are ahead, 42 against 50 us on 4 experts of 2048 x 1024).
+// mostly fit one, and for few rows in all (one expert of 2048 x 4096, 200 rows
+// 30 us against 39 with 128-row tiles; of 5120 x 8192, 320 rows 59 against 75,
+// 640 rows 80 against 83).  Near the line it goes either way: one of 7168 x
+// 2048, 640 rows 45 against 33; one of 2048 x 768, 800 rows 10 against 12.
 constexpr int kSmallAvgRows = 100;
 constexpr int kSmallMaxRows = 8192;
 inline int64_t small_rows64_max(int E) { return std::max<int64_t>(32 * (int64_t)E + 31, 768); }

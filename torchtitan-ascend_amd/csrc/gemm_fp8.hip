@@ -23,8 +23,8 @@
 //     form, with no partial sums kept across MFMAs.  A block's scale FMAs run
 //     under the next block's MFMAs, the last block's under the next stage's
 //     first, and with two waves per SIMD under the other wave's as well.
-//   * The 256 x 128 tile was bound by the L2 -> LDS stream (each CU keeps
-//     about 64 line requests in flight), so the tile is as large as the
+//   * The 256 x 128 tile was bound by its L2 -> LDS stream (about 64 line
+//     requests in flight per CU at ~450 cycles), so the tile is as large as the
 //     registers allow: 256 x 256 moves 66 KB per 16.8 MFLOP stage where
 //     256 x 128 moved 48 KB per 8.4.  With it a stage's DMA has landed
 //     before the barrier that needs it (~1 % of the stage waiting), and the

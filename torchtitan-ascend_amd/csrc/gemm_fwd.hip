@@ -30,10 +30,11 @@
 //     are therefore free early, and the next-but-one stage's DMAs into them
 //     are in flight for almost two stages; they go out one at a time between
 //     the MFMAs (run_tile).
-//   * What bounds it: at C3 w13 the k loop runs at 1.65-1.95 GHz (the chip
-//     lowers its clock under MFMA load) with the matrix cores ~73 % busy, the
-//     rest of a stage lost around its two barriers; without the DMAs the
-//     same loop holds 2.2 GHz.  Measured, one box, against 32x32x16 MFMAs
+//   * What bounds it: at C3 w13 the chip runs at 1.96 GHz (it lowers its
+//     clock under MFMA load) with the matrix cores 64 % busy over the launch
+//     (w2 59 %; C2, whose tiles have 32 and 12 stages, 54 and 42 %), the rest
+//     lost around a stage's two barriers, in the epilogues and in the last
+//     round.  Measured, one machine, against 32x32x16 MFMAs
 //     over k16 steps with each stage's DMAs issued in two bursts: C2 w13 401
 //     -> 381 us, w2 245 -> 235, dgrad + SwiGLU backward 344 -> 279; C3 w13
 //     1257 -> 1183, w2 676 -> 633, dgrad + SwiGLU backward 768 -> 699, dgrad
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
   const int nqt = sload_int(a.n_qtiles);
   const int ntiles = nqt * a.np_tiles;
   // (the schedule scalars are pinned to SGPRs: divisions are expanded in
-  // VALU, and the stage advance in issue_p must stay scalar)
+  // VALU, and issue_advance must stay scalar)
   auto U = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   const int ksteps = U(a.kred / TK);
   // Tail split: the walk has R full rounds of G tiles and rt tiles left
@@ -293,14 +294,16 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     }
     d_r = r;
   };
-  // A stage's DMA is issued in two parts: the weight rows (P) at the stage
-  // barrier that frees their buffer, the token rows (Q) one k16 step later
-  // (see the k loop).  issue_p sets the stage's bases, which issue_q reads.
+  // A stage's DMAs go out one instruction at a time between the MFMAs of the
+  // stage two before it, whose buffer they fill: the weight rows and the first
+  // QA token-row instructions after its barrier A, the other token rows after
+  // its barrier B (run_tile).  issue_prep sets the bases that issue_p1 and
+  // issue_q1 read, issue_advance steps to the next stage.
   uint64_t d_spb = 0, d_sqb = 0;
   uint32_t d_sst = 0;
-  // issue_p is called for stages 0, 1, 2, ... in order: the (unit, k stage)
-  // of the next one is advanced here rather than divided out per call.
-  // Past the end the last stage is issued again.
+  // Stages are issued in order, 0, 1, 2, ...: the (unit, k stage) of the next
+  // one is advanced rather than divided out per call.  Past the end the last
+  // stage is issued again.
   int n_r = 0, n_ks = nfull > 0 ? 0 : pc_k0, n_kend = nfull > 0 ? ksteps : pc_k1, n_left = total;
   auto issue_prep = [&](int s) {
     if (n_r != d_r) dma_tile(n_r);
@@ -329,9 +332,9 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
     }
   };
   auto issue_advance = [&]() {
-    // Advance to the next stage only now: whatever sits between the stage
-    // barrier and these DMAs delays every stage (the empty asm keeps the
-    // compiler from hoisting the update above them).  Selects, no branches.
+    // Advance to the next stage only after its DMAs: whatever sits between a
+    // barrier and the DMAs behind it delays every stage (the empty asm keeps
+    // the compiler from hoisting the update above them).  Selects, no branches.
     n_left = __builtin_amdgcn_readfirstlane(n_left);
     n_ks = __builtin_amdgcn_readfirstlane(n_ks);
     n_kend = __builtin_amdgcn_readfirstlane(n_kend);

@@ -7,9 +7,9 @@
 // expert's weights from HBM once, not by the MFMAs, and what the streaming
 // rate needs is requests in flight all the time: a copy of the weight stream
 // alone (LDS DMA, one workgroup per CU) reaches 6.1 TB/s with 64 KB in
-// flight per CU and 4.7 with 32 KB.  The 320 x 256 kernel (gemm_fwd.hip)
-// has two stages and waits for everything in flight at every stage barrier,
-// which is right for its compute-bound shapes and leaves 4.2-4.7 TB/s here.
+// flight per CU and 4.7 with 32 KB.  The 320 x 256 kernel (gemm_fwd.hip) holds
+// about one stage in flight across its barriers; with few tiles it leaves CUs
+// idle, and every tile of few rows costs it the time of 160.
 //
 // Tile: up to TQ (64 or 128) token rows x STP (128 or 256) weight rows, k in
 // stages of 64 (128-byte rows).  A ring of NS stages, one barrier per stage
@@ -31,11 +31,15 @@
 // a lane's accumulator groups g = 0, 2 are gate columns and g = 1, 3 the
 // matching up columns, and the activation needs no exchange.
 //
-// Measured (both GEMMs and the K-way sum, one MI355X): Qwen3-30B-A3B experts,
-// 32 tokens 243 -> 196 us (1.2 GB of weights: 6.0 TB/s in w13), 1003 tokens
-// 299 -> 251; DeepSeek-V3 shard of 32 experts, 200 rows 553 -> 470 us (w13
-// 6.0 TB/s); the 256 x 512 debug model's 2048 rows 44 -> 23 us (32 and 8
-// large tiles on 256 CUs before).
+// Measured, w13 / w2, us, against the 320 x 256 kernel: 64 experts of 768 x
+// 2048 (Qwen3-30B-A3B), 2 rows each 65 / 29 against 76 / 32, 64 rows 83 / 40
+// against 92 / 40; 128 of them a tie from 2 to 40 rows (127 / 66 and 152 / 89
+// against 129 / 69 and 147 / 88: 5.9-6.1 TB/s of weights on both); 32 of 7168
+// x 2048, 9 rows 306 / 166 against 307 / 179; the 256 x 512 debug model's 2000
+// rows 8 / 10 against 19 / 20 (32 and 8 large tiles on 256 CUs).  Against the
+// large kernel with one stage barrier for everything in flight, both GEMMs and
+// the K-way sum: 128 experts of 768 x 2048, 32 tokens 243 -> 196 us, 1003
+// tokens 299 -> 251; the shard of 32, 200 rows 553 -> 470.
 //
 // Reference semantics: torchtitanturbo/models/common/npu_gmm.py:17-38.
 #include "common.h"
@@ -63,7 +67,7 @@ struct Geo {
   static constexpr int IPW = SDMA_P + DMA_Q;  // DMAs per wave and stage
   static constexpr int NJ = TQ / 64;          // token blocks per wave
   static constexpr int STAGE = SP_BYTES + TQ * SROW;
-  static constexpr int RING = NS * STAGE;  // 144 KB / 128 KB
+  static constexpr int RING = NS * STAGE;  // 144 KB (64 x 128, 128 x 256), 120 KB (64 x 256), 128 KB (128 x 128)
   static constexpr int META = TQ * 8;      // destination rows, scales
   // gathered rows: per wave, two slots (tile round % 2) of DMA_Q x 64 ids
   static constexpr int IDS = SWAVES * 2 * DMA_Q * 256;
