@@ -1,7 +1,6 @@
-"""Benchmark of the MI355X MoE expert path (BASELINE.json metric).
+"""Benchmark of the MI355X MoE expert path.
 
-Default workload (Qwen3-30B-A3B shape, MoE layer
-forward, bf16): T=8192 tokens, D=2048, H=768, E=128 experts, top-8 softmax
+Default workload (Qwen3-30B-A3B shape, MoE layer forward, bf16): T=8192 tokens, D=2048, H=768, E=128 experts, top-8 softmax
 router with renormalised weights.  One step = router (gate GEMM split over D
 + fp32 softmax + top-k + renorm + histogram) -> stable sort + tile table ->
 grouped GEMM w13 + SwiGLU with the permute gather in its loads -> grouped

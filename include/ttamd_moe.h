@@ -537,9 +537,9 @@ int ttamd_grouped_mm_wgrad(const void* dy, const void* x, const int32_t* offs,
                            void* stream);
 
 /* ------------------------------------------------------------------------ *
- * fp8 e4m3 experts with fp32 block scales.               *
- * The reference has no fp8 path; these follow the published recipe the      *
- * north star names: scale = absmax / 448 per block, code = e4m3fn(v /       *
+ * fp8 e4m3 experts with fp32 block scales.                                  *
+ * The reference has no fp8 path; these follow the published recipe:         *
+ * scale = absmax / 448 per block, code = e4m3fn(v /                         *
  * scale) rounded to nearest even, value = code * scale, GEMM in fp32.      *
  * e4m3 is the OCP "fn" format (bias 7, max 448, 0x7f = NaN).  An all-zero   *
  * block has scale 0 and codes 0.  Inputs are finite.                        *

@@ -531,9 +531,9 @@ def expert_weight_grad_slices(routed: np.ndarray, dy: np.ndarray, w13_e: np.ndar
 
 
 # ---------------------------------------------------------------------------
-# fp8 e4m3 with block scales (not in the reference, which
-# has no fp8 path: the published recipe is restated -- s = absmax / 448 per
-# block, q = e4m3fn(v / s), dequantised value q * s, GEMM in fp32).
+# fp8 e4m3 with block scales (not in the reference, which has no fp8 path:
+# the published recipe is restated -- s = absmax / 448 per block,
+# q = e4m3fn(v / s), dequantised value q * s, GEMM in fp32).
 # ---------------------------------------------------------------------------
 FP8_MAX = 448.0
 FP8_BLOCK = 128
@@ -641,7 +641,7 @@ def grouped_mm_fp8(xq, sx, wq, sw, offs) -> np.ndarray:
 
 def moe_forward_fp8(x, top_scores, idx, w13q, s13, w2q, s2, num_experts, score_before_experts,
                     swiglu_limit=None):
-    """moe_forward with fp8 experts (BASELINE config 5): the dispatched rows
+    """moe_forward with fp8 experts: the dispatched rows
     are quantised per token and 128 channels, w13/w2 are pre-quantised with
     128 x 128 block scales, h and a are materialised in bf16 as in the bf16
     path, and the SwiGLU output is re-quantised per row for the w2 GEMM."""

@@ -1,4 +1,4 @@
-"""BASELINE config 3 at full size: the Llama4-Scout-shaped MoE layer forward
+"""Full size: the Llama4-Scout-shaped MoE layer forward
 + backward (T=8192, D=5120, H=8192, E=16, top-1 sigmoid router, score before
 the experts, plus one always-on shared expert of the same shape), through
 the converted HipGroupedExperts layer and the shared-expert combine, with

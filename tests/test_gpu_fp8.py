@@ -1,4 +1,4 @@
-"""GPU parity of the fp8 e4m3 path (BASELINE config 5) against the CPU oracle.
+"""GPU parity of the fp8 e4m3 path against the CPU oracle.
 
 Quantisation is byte work derived from floats: codes and scales must be
 bit-exact.  The fp8 GEMMs read the same codes and scales as the oracle, whose

@@ -1,7 +1,7 @@
 """The inference layer captured as one HIP graph (graph.MoELayerGraph):
 every replay equals the eager two-call step on the same input, bit for bit,
 with eager work and synchronisations between the replays (replays after the
-first are where wrong graph nodes would show).  Shapes
+first are where wrong graph nodes would show).  Shapes: the debug layer
 (Llama4-debugmodel: T=2048, D=256, H=512, E=8, top-1 sigmoid, score before
 the experts), a reduced Qwen3-30B-A3B layer (top-8 softmax + renorm) and a
 layer whose w13 leftover tiles are split along k.

@@ -1,6 +1,6 @@
 """GPU parity of the whole converted MoE expert layer (dispatch -> experts ->
 combine) against the CPU oracle, forward and backward, including the
-BASELINE configs at full size (checked on sampled tokens)."""
+full-size workloads (checked on sampled tokens)."""
 from __future__ import annotations
 
 import importlib

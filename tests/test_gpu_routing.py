@@ -41,7 +41,7 @@ def test_route_golden(ops, name):
 @pytest.mark.parametrize(
     "T,K,E,dtype",
     [
-        (8192, 8, 128, torch.int64),  # Qwen3-30B-A3B shape (BASELINE config 2)
+        (8192, 8, 128, torch.int64),  # Qwen3-30B-A3B shape
         (8192, 8, 128, torch.int32),
         (2048, 1, 8, torch.int64),  # Llama4 debug (config 1)
         (8192, 1, 16, torch.int64),  # Llama4 Scout (config 3)

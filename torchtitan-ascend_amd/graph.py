@@ -4,7 +4,7 @@ A step of the layer is two C-ABI calls (ttamd_router_route, then
 ttamd_moe_experts_forward: six kernel launches, all on the caller's
 stream, none of them a memset, a host synchronisation or an allocation
 inside the library).  At small shapes the host's cost per call exceeds
-the kernels' run time (T = 2048, D = 256), so the pair
+the kernels' run time (the debug shape: T = 2048, D = 256), so the pair
 is recorded once with torch's graph capture over that stream and replayed:
 one launch per step.  Every buffer the step uses (the routing outputs, the
 tile plan, the workspaces, the output) is allocated once, during capture,
