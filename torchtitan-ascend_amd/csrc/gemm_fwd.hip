@@ -378,9 +378,9 @@ __global__ __launch_bounds__(FTHREADS, 1) void gg_fwd_kernel(const FwdArgs a) {
   // t, 2 + t, 4 + t and 6 + t, the same for both operands: with neighbouring
   // chunks (4 t + l / 16) the reads of 16 rows meet on the same LDS banks
   // (measured 300 B/ns per CU against 555, as the 32-row reads).
-  // (The 32x32x16 form moves twice the accumulators per flop and, at the
-  // chip's power limit, runs at a lower clock: the k loop alone on random
-  // operands 1565 TFLOP/s against 1750.)
+  // (The 32x32x16 form moves twice the accumulators per flop and runs at a
+  // lower clock: the k loop alone, fragment reads included, on random operands
+  // 1565 TFLOP/s against 1750; a second measurement of the latter 1629-1715.)
   const int r16 = l & 15;
   const int g4 = l >> 4;
   const int fa = cswz(r16);

@@ -14,8 +14,8 @@
 //     group, so fp32 / bf16 results leave as 16- / 8-byte stores).
 //   * 8 waves (2 per SIMD), 2 (n) x 4 (k); each wave 128 n x 64 k =
 //     4 x 8 accumulators of v_mfma_f32_16x16x32_bf16 (half the accumulator
-//     traffic per flop of the 32x32x16 form and, at the chip's power limit,
-//     a ~12 % higher MFMA rate).
+//     traffic per flop of the 32x32x16 form and, under the clock that the
+//     load leaves, a 4-12 % higher MFMA rate).
 //   * Stages of 64 rows m: x rows (64 x 512 bytes) and dy rows (64 x 512
 //     bytes) DMA'd by global_load_lds_dwordx4 into two 64 KB buffers, chunk
 //     c of row m stored at c ^ ptswz(m) (conflict-free transposed reads).
